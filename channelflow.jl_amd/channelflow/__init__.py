@@ -491,7 +491,7 @@ def FFT(problem, u):
     torch = _torch()
     single = u.dim() == 3
     uu = u.unsqueeze(0) if single else u
-    out = g.zeros_spec(uu.shape[0])
+    out = torch.empty((uu.shape[0],) + g.spec_shape, dtype=torch.complex128, device="cuda")  # every mode is written
     if uu.dtype != torch.float64 or tuple(uu.shape[1:]) != g.phys_shape:
         raise DimensionMismatch("forward transform requires padded physical input")
     if uu.shape[0] == 3:  # one launch per pass for the vector field
@@ -510,7 +510,7 @@ def IFFT(problem, U):
     g = problem.grid
     single = U.dim() == 3
     UU = U.unsqueeze(0) if single else U
-    out = g.zeros_phys(UU.shape[0])
+    out = _torch().empty((UU.shape[0],) + g.phys_shape, dtype=_torch().float64, device="cuda")  # every point is written
     if UU.shape[0] == 3:  # one launch per pass for the vector field
         srcs = [UU[c].contiguous() for c in range(3)]
         for src in srcs:

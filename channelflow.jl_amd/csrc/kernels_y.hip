@@ -858,53 +858,95 @@ __global__ void __launch_bounds__(YNT) ydivergence_kernel(YArgs a) {
 // excluded.  Y_DOT: sum over the three components of U (U) and V (Rin).
 // Y_DISSIPATION: u = v = curl U (operators.jl:172-190); the caller scales by nu.
 // Each block writes its partial sum to partial[blockIdx.x].
+//
+// Bound by FP64 issue of the Ny^2/2 products per component.  M is Toeplitz +
+// Hankel, so a lane needs mu only at m + n and m - n: with n = K q + f (f
+// unrolled) both are entries at a fixed residue mod K and at the quotients
+// t + q, t - q, one new entry a residue and iteration (the other is the
+// previous iteration's).  The table holds mu/2 by residue, so the lanes of a
+// group read consecutive words, and it takes the place of the per-degree
+// constants, which this kernel does not use.  The three components share the
+// entries.  At 128x97x128: 225 us with two divisions per entry, 38.6 us so.
 template <int L, int K>
 __global__ void __launch_bounds__(YNT) ydot_kernel(YArgs a, int curl) {
     extern __shared__ double2 smem[];
-    load_tables<L, K>(smem, a);
+    constexpr int NT = K * L, LT = 3 * L;  // entries i = -NT .. 2 NT - 1 at [i mod K][i / K + L]
+    double* mu = reinterpret_cast<double*>(smem + a.dct.n);
+    for (int j = threadIdx.x; j < 3 * NT; j += YNT) {
+        const int i = j - NT;
+        mu[(j % K) * LT + j / K] = (i % 2 == 0) ? 0.5 / (1.0 - (double)i * i) : 0.0;
+    }
+    __syncthreads();
     Tile<L, K> tile(a.gd, smem, a.dct.n, a.ld, y_region_slots<L, K>(a.ld), blockIdx.x);
     Group<L, K> g(tile.tab);
     ModeInfo mi = mode_info(a.gd, tile.s);
     const int Ny = a.gd.Ny;
-    double2* vline = tile.stash;  // this group's copy of v, indexed by degree
-    CVec<K> W0, W1, W2;
+    double2* vline = tile.stash;  // this group's copies of v, indexed by degree
+    CVec<K> u[3];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) u[c] = tile.load(a.U[c], g);
     if (curl) {
-        CVec<K> U0 = tile.load(a.U[0], g), U1 = tile.load(a.U[1], g), U2 = tile.load(a.U[2], g);
-        CVec<K> d2 = cheb_deriv(g, U2), d0 = cheb_deriv(g, U0);
+        const CVec<K> d2 = cheb_deriv(g, u[2]), d0 = cheb_deriv(g, u[0]);
 #pragma unroll
         for (int e = 0; e < K; ++e) {
-            W0.v[e] = csub(d2.v[e], cmuli(cscale(U1.v[e], mi.kz)));
-            W1.v[e] = cmuli(csub(cscale(U0.v[e], mi.kz), cscale(U2.v[e], mi.kx)));
-            W2.v[e] = csub(cmuli(cscale(U1.v[e], mi.kx)), d0.v[e]);
+            const double2 w0 = csub(d2.v[e], cmuli(cscale(u[1].v[e], mi.kz)));
+            const double2 w1 = cmuli(csub(cscale(u[0].v[e], mi.kz), cscale(u[2].v[e], mi.kx)));
+            const double2 w2 = csub(cmuli(cscale(u[1].v[e], mi.kx)), d0.v[e]);
+            u[0].v[e] = w0;
+            u[1].v[e] = w1;
+            u[2].v[e] = w2;
+        }
+#pragma unroll
+        for (int c = 0; c < 3; ++c) stash(vline + c * NT, g, u[c]);
+    } else {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) stash(vline + c * NT, g, tile.load(a.Rin[c], g));
+    }
+    wave_sync();
+    double2 s[3][K];
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+#pragma unroll
+        for (int e = 0; e < K; ++e) s[c][e] = czero();
+    // plus[r] = mu/2 at m + n = K (t + q) + r and K (t + q + 1) + r, minus[r]
+    // at m - n = K (t - q - 1) + r and K (t - q) + r (even r)
+    double plus[2][K], minus[2][K];
+#pragma unroll
+    for (int r = 0; r < K; r += 2) {
+        plus[0][r] = mu[r * LT + L + g.t];
+        minus[1][r] = mu[r * LT + L + g.t];
+    }
+    const int nq = (Ny + K - 1) / K;
+#pragma unroll 1
+    for (int q = 0; q < nq; ++q) {
+#pragma unroll
+        for (int r = 0; r < K; r += 2) {
+            plus[1][r] = mu[r * LT + L + g.t + q + 1];
+            minus[0][r] = mu[r * LT + L + g.t - q - 1];
+        }
+#pragma unroll
+        for (int f = 0; f < K; ++f) {
+            double2 v[3];
+#pragma unroll
+            for (int c = 0; c < 3; ++c) v[c] = vline[c * NT + K * q + f];
+#pragma unroll
+            for (int e = f & 1; e < K; e += 2) {
+                const double Mmn = plus[(e + f) / K][(e + f) % K] + (e >= f ? minus[1][e >= f ? e - f : 0] : minus[0][e >= f ? 0 : K + e - f]);
+#pragma unroll
+                for (int c = 0; c < 3; ++c) s[c][e] = cfma(Mmn, v[c], s[c][e]);
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < K; r += 2) {
+            plus[0][r] = plus[1][r];
+            minus[1][r] = minus[0][r];
         }
     }
     double acc = 0.0;
-#pragma unroll 1
-    for (int c = 0; c < 3; ++c) {
-        CVec<K> u, v;
-        if (curl) {
-            u = (c == 0) ? W0 : (c == 1) ? W1 : W2;
-            v = u;
-        } else {
-            u = tile.load(a.U[c], g);
-            v = tile.load(a.Rin[c], g);
-        }
-        stash(vline, g, v);
-        wave_sync();
 #pragma unroll
-        for (int e = 0; e < K; ++e) {
-            const int m = K * g.t + e;
-            double2 s = czero();
-            if (m < Ny)
-                for (int n = m & 1; n < Ny; n += 2) {
-                    const double kp = m + n, km = m - n;
-                    const double Mmn = 0.5 * (1.0 / (1.0 - kp * kp) + 1.0 / (1.0 - km * km));
-                    s = cfma(Mmn, vline[n], s);
-                }
-            acc += u.v[e].x * s.x + u.v[e].y * s.y;  // Re(conj(u_m) (M v)_m)
-        }
-        wave_sync();
-    }
+    for (int c = 0; c < 3; ++c)
+#pragma unroll
+        for (int e = 0; e < K; ++e) acc += u[c].v[e].x * s[c][e].x + u[c].v[e].y * s[c][e].y;  // Re(conj(u_m) (M v)_m)
     acc = g.sum(acc);
     const bool use = mi.valid && !mi.nyq;
     double* part = reinterpret_cast<double*>(smem);  // twiddle area is free now
@@ -997,16 +1039,30 @@ __global__ void __launch_bounds__(YNT) ystats_kernel(YArgs a) {
 }
 
 #if CF_Y_PART == 0
-__global__ void __launch_bounds__(256) reduce_columns_kernel(const double* part, int nblocks, int nq, double* out) {
-    const int q = blockIdx.x * 256 + threadIdx.x;
-    if (q >= nq) return;
-    double s = 0.0;
-    for (int b = 0; b < nblocks; ++b) s += part[(size_t)b * nq + q];
-    out[q] = s;
+// Column sums of the blocks' partials in a fixed order: a block owns 32
+// columns, its 32 row groups sum every 32nd row and are added in order.
+// Bound by the latency of the loads: one thread per column took 254 us for the
+// 1040 x 873 partials of 128x97x128, all rows in one serial chain; 7.6 us so.
+constexpr int RCOL = 32, RGRP = 32;
+__global__ void __launch_bounds__(RCOL * RGRP) reduce_columns_kernel(const double* part, int nblocks, int nq, double* out) {
+    __shared__ double s[RGRP][RCOL];
+    const int c = threadIdx.x % RCOL, r = threadIdx.x / RCOL, q = blockIdx.x * RCOL + c;
+    double v = 0.0;
+    if (q < nq) {
+#pragma unroll 8
+        for (int b = r; b < nblocks; b += RGRP) v += part[(size_t)b * nq + q];
+    }
+    s[r][c] = v;
+    __syncthreads();
+    if (r == 0 && q < nq) {
+        for (int i = 1; i < RGRP; ++i) v += s[i][c];
+        out[q] = v;
+    }
 }
 
 hipError_t launch_reduce_columns(const double* part, int nblocks, int nq, double* out, hipStream_t st) {
-    hipLaunchKernelGGL(reduce_columns_kernel, dim3((unsigned)((nq + 255) / 256)), dim3(256), 0, st, part, nblocks, nq, out);
+    hipLaunchKernelGGL(reduce_columns_kernel, dim3((unsigned)((nq + RCOL - 1) / RCOL)), dim3(RCOL * RGRP), 0, st, part,
+                       nblocks, nq, out);
     return hipGetLastError();
 }
 
