@@ -93,6 +93,7 @@ struct cf_problem {
     int KT = 1, zld = 0, LPB = 1, xld = 0, yld = 0;
     int xwaves = 4;  // even Nxp: wavefronts per block of the nonlinear x pass
     int zppt = 0;    // z pass in-place points per thread (0: two buffers)
+    int zr1 = 0, zr2 = 0;  // register radices of the FP64 z pass (0: none, the staged passes)
     int xppt = 0;    // even-Nxp x pass in-place points per lane (0: two buffers)
     // forcing(tstage, U, F) hook: host callback and the caller's F fields
     cf_forcing_fn force_fn = nullptr;
@@ -297,6 +298,18 @@ static void free_all(cf_problem* h) {
     h->allocs.clear();
 }
 
+// z tile widths that a caller may set: an in-place width (one LDS buffer) or,
+// for plans that need two buffers, a width whose two buffers fit 64 KB
+static bool z_width_ok(cf_problem* h, int kt) {
+    ZArgs z;
+    std::memset(&z, 0, sizeof(z));
+    z.gd = h->gd;
+    z.KT = kt;
+    z.ld = h->zld;
+    z.ppt = z_inplace_ppt(h->pz, kt);
+    return (z.ppt || kt <= 16) && z_lds_bytes(z) <= 64 * 1024;
+}
+
 extern "C" const char* cf_last_error(void) { return g_err.c_str(); }
 
 extern "C" int cf_problem_create(const cf_config* cfg, cf_problem** out) {
@@ -340,7 +353,9 @@ extern "C" int cf_problem_create(const cf_config* cfg, cf_problem** out) {
     gd.P = cfg->Ny - 1;
     gd.B = (long long)gd.Nxh * gd.Nz;
     gd.S = gd.B * gd.Ny;
-    gd.Sz = (long long)gd.Nxh * gd.Nzp * gd.Ny;
+    gd.nk = (cfg->Nx % 2 == 0) ? cfg->Nx / 2 : gd.Nxh;
+    gd.ldk = gd.nk >= 32 ? (gd.nk + 7) / 8 * 8 : (gd.nk + 3) / 4 * 4;  // 128-byte rows; 64-byte ones where the pad would show
+    gd.Sz = (long long)gd.ldk * gd.Nzp * gd.Ny;
     gd.alpha = 2.0 * M_PI / cfg->Lx;
     gd.beta = 2.0 * M_PI / cfg->Lz;
     h->Lx = cfg->Lx;
@@ -387,6 +402,7 @@ extern "C" int cf_problem_create(const cf_config* cfg, cf_problem** out) {
     // plans
     if ((rc = make_plan(h, gd.Nzp, h->pz))) return bail(rc);
     if ((rc = make_plan(h, 2 * gd.P, h->py))) return bail(rc);
+    (void)z_reg_split(gd.Nzp, &h->zr1, &h->zr2);
     int M = (gd.Nxp % 2 == 0) ? gd.Nxp / 2 : gd.Nxp;
     if ((rc = make_plan(h, M, h->px))) return bail(rc);
     {
@@ -408,6 +424,17 @@ extern "C" int cf_problem_create(const cf_config* cfg, cf_problem** out) {
     if (!h->zppt) {
         h->KT = (int)std::max<size_t>(1, std::min<size_t>(16, LDS_MAX / (2 * (size_t)h->zld * sizeof(double2))));
         h->KT = std::min(h->KT, gd.Nxh);
+    }
+    if (h->zr1) {
+        // register passes: 256-byte column segments; narrower tiles where the
+        // launch would leave CUs without a block, or three blocks would not
+        // share a CU's LDS
+        h->KT = 16;
+        auto blocks = [&](int kt) { return (long long)((gd.nk + kt - 1) / kt) * gd.Ny * 6; };
+        while (h->KT > 4 && (blocks(h->KT) < 512 || (size_t)gd.Nzp * (h->KT + 1) * sizeof(double2) > 53 * 1024)) h->KT /= 2;
+        h->KT = std::min(h->KT, gd.Nxh);
+        while (h->KT > 1 && !z_width_ok(h, h->KT)) --h->KT;
+        h->zppt = z_inplace_ppt(h->pz, h->KT);
     }
     h->xld = M + 1;
     {
@@ -550,6 +577,8 @@ static ZArgs make_zargs(cf_problem* h, int nf, double2* const* in, double2* cons
     z.nfields = nf;
     z.ppt = mixed ? h->zppt32 : h->zppt;
     z.mixed = mixed ? 1 : 0;
+    z.r1 = mixed ? 0 : h->zr1;
+    z.r2 = mixed ? 0 : h->zr2;
     z.dz_mask = dz_mask;
     z.mul_kt = recip_mul((unsigned)z.KT);
     for (int i = 0; i < nf; ++i) {
@@ -577,7 +606,7 @@ static XArgs base_xargs(cf_problem* h, bool mixed = false) {
     x.ppt = mixed ? h->xppt32 : h->xppt;
     x.mixed = mixed ? 1 : 0;
     x.mul_m = recip_mul((unsigned)std::max(1, h->gd.Nxp / 2));
-    x.mul_nxh = recip_mul((unsigned)h->gd.Nxh);
+    x.mul_nk = recip_mul((unsigned)h->gd.nk);
     x.mul_nx = recip_mul((unsigned)(std::max(1, h->gd.Nxp / 2) + 1));
     return x;
 }
@@ -601,7 +630,11 @@ struct NonlinearArgs {
     XArgs x;
 };
 
-static NonlinearArgs nonlinear_args(cf_problem* h, bool mixed) {
+// staged: the z passes of the setup calls (cf_nonlinear, cf_pressure) keep the
+// staged multi-pass transforms.  An FP32-mixed run amplifies a last-bit change
+// of its initial pressure to FP32 noise within one step, so the calls that
+// prepare it keep their bits; they run once per trajectory.
+static NonlinearArgs nonlinear_args(cf_problem* h, bool mixed, bool staged = false) {
     const GridDims& gd = h->gd;
     double2* six[6];
     double2* zb[9];
@@ -642,11 +675,14 @@ static NonlinearArgs nonlinear_args(cf_problem* h, bool mixed) {
     }
     const int nout = h->form == CF_FORM_DIVERGENCE ? 6 : 3;
     na.zout = make_zargs(h, nout, zb, six, 0, mixed);
+    if (staged)
+        for (ZArgs* z : {&na.zin, &na.zout}) z->r1 = z->r2 = 0;
     return na;
 }
 
-static int enqueue_nonlinear_phys(cf_problem* h, hipStream_t st, Timer* tm = nullptr, bool mixed = false) {
-    const NonlinearArgs na = nonlinear_args(h, mixed);
+static int enqueue_nonlinear_phys(cf_problem* h, hipStream_t st, Timer* tm = nullptr, bool mixed = false,
+                                  bool staged = false) {
+    const NonlinearArgs na = nonlinear_args(h, mixed, staged);
     HIPTRY(launch_zpass(+1, na.zin, st));
     if (int rc = tmark(tm, 1, st)) return rc;
     HIPTRY(launch_xpass(na.x, st));
@@ -1345,7 +1381,7 @@ extern "C" int cf_inverse3(cf_problem* h, const double* U0, const double* U1, co
 // nonlinear term of U into spectral N (3 fields)
 static int enqueue_nonlinear_spec(cf_problem* h, double2* const U[3], double2* const N[3], hipStream_t st) {
     if (int rc = enqueue_prologue(h, U, st)) return rc;
-    if (int rc = enqueue_nonlinear_phys(h, st)) return rc;
+    if (int rc = enqueue_nonlinear_phys(h, st, nullptr, false, true)) return rc;
     if (h->form == CF_FORM_DIVERGENCE) return enqueue_nonlinear_coef(h, N, st);
     YArgs a = base_yargs(h);
     a.nl_sign = (h->form == CF_FORM_CONVECTIVE) ? -1.0 : 1.0;
@@ -1641,17 +1677,8 @@ extern "C" int cf_problem_tune(cf_problem* h, void* stream) {
     float best = 1e30f;
     for (int kt = 1; kt <= std::min(32, h->gd.Nxh) && !rc; ++kt) {
         const int ppt = z_inplace_ppt(h->pz, kt);
-        if (!ppt && !(kt == keepKT && keepPPT == 0)) continue;
-        if (z_lds_bytes([&] {
-                ZArgs z;
-                std::memset(&z, 0, sizeof(z));
-                z.gd = h->gd;
-                z.KT = kt;
-                z.ld = h->zld;
-                z.ppt = ppt;
-                return z;
-            }()) > 64 * 1024)
-            continue;
+        if (!h->zr1 && !ppt && !(kt == keepKT && keepPPT == 0)) continue;
+        if (!z_width_ok(h, kt)) continue;
         h->KT = kt;
         h->zppt = ppt;
         const NonlinearArgs na = nonlinear_args(h, false);
@@ -1852,7 +1879,7 @@ enum { B_YPRO = 0, B_ZINV, B_X, B_ZFWD, B_YSTAGE };
 
 struct BatchLaunch {
     int cls;        // B_*
-    int tp, waves;  // template parameter (L or in-place width), x wavefronts per block
+    int tp, waves;  // template parameter (L, in-place width or z register class), wavefronts per block (x, register z)
     int mode;       // x form
     const void* tab;
     const unsigned* start;
@@ -1895,8 +1922,12 @@ static hipError_t run_batch(const BatchLaunch& b, hipStream_t st) {
     switch (b.cls) {
         case B_YPRO: return launch_ykernel_batch(Y_PROLOGUE, b.tp, (const YArgs*)b.tab, b.start, b.n, b.nblocks, b.lds, st);
         case B_YSTAGE: return launch_ykernel_batch(Y_STAGE, b.tp, (const YArgs*)b.tab, b.start, b.n, b.nblocks, b.lds, st);
-        case B_ZINV: return launch_zpass_batch(+1, b.tp, (const ZArgs*)b.tab, b.start, b.n, b.nblocks, b.lds, st);
-        case B_ZFWD: return launch_zpass_batch(-1, b.tp, (const ZArgs*)b.tab, b.start, b.n, b.nblocks, b.lds, st);
+        case B_ZINV:
+        case B_ZFWD: {
+            const int dir = b.cls == B_ZINV ? +1 : -1;
+            if (b.waves) return launch_zreg_batch(dir, b.tp, 64 * b.waves, (const ZArgs*)b.tab, b.start, b.n, b.nblocks, b.lds, st);
+            return launch_zpass_batch(dir, b.tp, (const ZArgs*)b.tab, b.start, b.n, b.nblocks, b.lds, st);
+        }
         case B_X: return launch_xpass_batch(b.mode, b.tp, b.waves, (const XArgs*)b.tab, b.start, b.n, b.nblocks, b.lds, st);
         default: return hipErrorInvalidValue;
     }
@@ -1987,10 +2018,13 @@ static int ens_build(cf_ensemble* e, std::vector<BatchLaunch>& step) {
         b = y_blocks(a.gd);
         l = y_lds_bytes(a.gd.Ny, a.ld);
     };
-    auto zkey = [](const ZArgs& a) { return std::array<int, 3>{a.ppt, 0, 0}; };
+    // register z passes: one launch per register class and block size
+    auto zkey = [](const ZArgs& a) {
+        return a.r1 ? std::array<int, 3>{z_reg_class(a), z_reg_threads(a) / 64, 0} : std::array<int, 3>{a.ppt, 0, 0};
+    };
     auto zinfo = [](const ZArgs& a, unsigned& b, size_t& l) {
         b = z_blocks(a);
-        l = z_lds_bytes(a);
+        l = a.r1 ? z_reg_lds(a) : z_lds_bytes(a);
     };
     auto xkey = [](const XArgs& a) { return std::array<int, 3>{a.ppt, a.waves, a.mode}; };
     auto xinfo = [](const XArgs& a, unsigned& b, size_t& l) {
@@ -2056,7 +2090,7 @@ static int ens_tune(cf_ensemble* e) {
         float best = 1e30f;
         for (int kt = 1; kt <= std::min(16, h->gd.Nxh); kt *= 2) {
             const int ppt = z_inplace_ppt(h->pz, kt);
-            if (!ppt) continue;
+            if (h->zr1 ? !z_width_ok(h, kt) : !ppt) continue;
             for (int i : members) {
                 e->tiles[i].KT = kt;
                 e->tiles[i].zppt = ppt;

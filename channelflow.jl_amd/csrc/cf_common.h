@@ -29,9 +29,13 @@ __host__ __device__ __forceinline__ unsigned fast_div(unsigned x, unsigned long 
 
 // Grid sizes (src/grids.jl:22-74): resolved (Nx, Ny, Nz), padded Nxp, Nzp,
 // half spectrum Nxh; P = Ny - 1; B = Nxh*Nz modes; S = B*Ny coefficients.
+// The z-padded workspace (k, zp, y) holds only the nk wavenumbers that the x
+// pass reads (no Nyquist column), its rows ldk >= nk apart: whole cache lines,
+// where rows of Nxh = Nx/2 + 1 straddle them.
 struct GridDims {
     int Nx, Ny, Nz, Nxh, Nxp, Nzp, P;
-    long long B, S, Sz;  // Sz = Nxh*Nzp*Ny (z-padded x-half spectrum)
+    int nk, ldk;
+    long long B, S, Sz;  // Sz = ldk*Nzp*Ny (z-padded x-half spectrum)
     double alpha, beta;  // 2 pi / Lx, 2 pi / Lz
 };
 

@@ -83,6 +83,7 @@ struct ZArgs {
     unsigned dz_mask;  // bit f: inverse pass multiplies field f by i*beta*l (z derivative)
     unsigned long long mul_kt;  // recip_mul(KT): index splits without integer division
     int mixed;                  // 1: fields are FP32 complex (float2) in the same buffers; in-place plans only
+    int r1, r2;                 // > 0: register radices, Nzp = r1 r2 (z_reg_split; FP64), else the staged passes
     const double2* in[9];
     double2* out[9];
 };
@@ -102,9 +103,9 @@ struct XArgs {
     int LPB, ld, mode, nfields;
     int waves;             // even Nxp: wavefronts (lines) per block, 1..4
     int ppt;               // even Nxp: in-place FFT points per lane (one LDS buffer), 0: two buffers
-    unsigned long long mul_m, mul_nxh, mul_nx;  // recip_mul of Nxp/2, Nxh and Nxp/2+1 (index splits)
+    unsigned long long mul_m, mul_nk, mul_nx;  // recip_mul of Nxp/2, nk and Nxp/2+1 (index splits)
     int mixed;             // 1: in/out are FP32 complex (float2); even Nxp, in-place wave path only
-    const double2* in[9];  // (k, zp, y) complex, Nxh per line
+    const double2* in[9];  // (k, zp, y) complex, nk per line of ldk
     double2* out[6];
     const double* rin[3];  // (x, zp, y) real
     double* rout[9];       // (x, zp, y) real outputs (X_INVERSE; X_GRADIENT: dV_i/dx_j at 3 i + j)
@@ -171,6 +172,14 @@ size_t y_lds_bytes(int Ny, int ld);
 hipError_t launch_zpass(int dir, const ZArgs& a, hipStream_t st);
 size_t z_lds_bytes(const ZArgs& a);
 int z_inplace_ppt(const FFTPlan& plan, int KT);  // 0: the plan needs two buffers
+bool reg_radix(int r);                           // radices built in registers
+bool z_reg_split(int n, int* r1, int* r2);       // false: n = r1 r2 has no such split
+hipError_t launch_zreg(int dir, const ZArgs& a, hipStream_t st);
+int z_reg_class(const ZArgs& a);    // register class of the kernel: radices up to 12, 16 or 24
+int z_reg_threads(const ZArgs& a);  // threads per block
+size_t z_reg_lds(const ZArgs& a);
+hipError_t launch_zreg_batch(int dir, int cls, int nthreads, const ZArgs* tab, const unsigned* start, int n,
+                             unsigned nblocks, size_t lds, hipStream_t st);
 hipError_t launch_xpass(const XArgs& a, hipStream_t st);
 size_t x_lds_bytes(const XArgs& a);
 int x_phys_lines(int mode);  // physical lines per (zp, y) line of the odd-Nxp x pass

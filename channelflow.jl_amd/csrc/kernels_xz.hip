@@ -37,14 +37,14 @@ __device__ __forceinline__ void zpass_body(const ZArgs& a, unsigned lb) {
     const int KT = a.KT, ld = a.ld;
     C* bufA = smem;
     C* bufB = smem + KT * ld;
-    const unsigned ntiles = (unsigned)((gd.Nxh + KT - 1) / KT);
+    const unsigned ntiles = (unsigned)((gd.nk + KT - 1) / KT);
     const unsigned tile = lb % ntiles, plane = lb / ntiles;
     const int y = (int)(plane % (unsigned)gd.Ny), f = (int)(plane / (unsigned)gd.Ny);
     const int k0 = (int)tile * KT;
     const int tid = threadIdx.x;
-    const int Nz = gd.Nz, Nzp = gd.Nzp, Nxh = gd.Nxh;
+    const int Nz = gd.Nz, Nzp = gd.Nzp, Nxh = gd.Nxh, nk = gd.nk, ldk = gd.ldk;
     const int npos = (Nz >> 1) + 1, nneg = Nz - npos;
-    const bool xeven = (gd.Nx % 2 == 0), zeven = (Nz % 2 == 0);
+    const bool zeven = (Nz % 2 == 0);
     const C zero = cplx<C>(T(0), T(0));
     if constexpr (PPT > 0)  // in-place mode: the second buffer holds the twiddle table
         for (int i = tid; i < Nzp; i += ZNT) bufB[i] = from_c64<C>(a.plan.tw[i]);
@@ -67,7 +67,7 @@ __device__ __forceinline__ void zpass_body(const ZArgs& a, unsigned lb) {
                 if (idx < total) {
                     int z = (int)fast_div((unsigned)idx, a.mul_kt), kk = idx - z * KT;
                     int k = k0 + kk;
-                    if (k < Nxh && !(xeven && k == gd.Nx / 2)) {
+                    if (k < nk) {
                         int l = -1;
                         if (z < npos) l = (zeven && z == Nz / 2) ? -1 : z;
                         else if (z >= Nzp - nneg) l = npos + (z - (Nzp - nneg));
@@ -88,7 +88,7 @@ __device__ __forceinline__ void zpass_body(const ZArgs& a, unsigned lb) {
             }
         }
     } else {
-        const C* in = reinterpret_cast<const C*>(a.in[f]) + (size_t)Nxh * Nzp * y;
+        const C* in = reinterpret_cast<const C*>(a.in[f]) + (size_t)ldk * Nzp * y;
         for (int base = tid; base < total; base += ZLOADS * ZNT) {
             C v[ZLOADS];
 #pragma unroll
@@ -98,7 +98,7 @@ __device__ __forceinline__ void zpass_body(const ZArgs& a, unsigned lb) {
                 if (idx < total) {
                     int z = (int)fast_div((unsigned)idx, a.mul_kt), kk = idx - z * KT;
                     int k = k0 + kk;
-                    if (k < Nxh) v[b] = in[k + (size_t)Nxh * z];
+                    if (k < nk) v[b] = in[k + (size_t)ldk * z];
                 }
             }
 #pragma unroll
@@ -116,11 +116,11 @@ __device__ __forceinline__ void zpass_body(const ZArgs& a, unsigned lb) {
     if constexpr (PPT > 0) lds_fft_inplace<PPT, false>(bufA, a.plan, (const C*)bufB, KT, ld, DIR, tid, ZNT);  // bufB: twiddles
     else res = lds_fft(bufA, bufB, a.plan, KT, ld, DIR, tid, ZNT);
     if (DIR > 0) {
-        C* out = reinterpret_cast<C*>(a.out[f]) + (size_t)Nxh * Nzp * y;
+        C* out = reinterpret_cast<C*>(a.out[f]) + (size_t)ldk * Nzp * y;
         for (int idx = tid; idx < KT * Nzp; idx += ZNT) {
             int z = (int)fast_div((unsigned)idx, a.mul_kt), kk = idx - z * KT;
             int k = k0 + kk;
-            if (k < Nxh) out[k + (size_t)Nxh * z] = res[kk * ld + z];
+            if (k < nk) out[k + (size_t)ldk * z] = res[kk * ld + z];
         }
     } else {
         C* out = reinterpret_cast<C*>(a.out[f]) + (size_t)Nxh * Nz * y;
@@ -128,7 +128,7 @@ __device__ __forceinline__ void zpass_body(const ZArgs& a, unsigned lb) {
             int l = (int)fast_div((unsigned)idx, a.mul_kt), kk = idx - l * KT;
             int k = k0 + kk;
             int z = (l < npos) ? l : Nzp - nneg + (l - npos);
-            if (k < Nxh) out[k + (size_t)Nxh * l] = res[kk * ld + z];
+            if (k < nk) out[k + (size_t)Nxh * l] = res[kk * ld + z];
         }
     }
 }
@@ -225,16 +225,15 @@ struct XCtx {
     // rotating form's Omega_y line)
     __device__ __forceinline__ void c2r(const double2* __restrict__ in, double* phys, bool dx = false,
                                         const double2* __restrict__ sub = nullptr) {
-        const bool xeven = (a.gd.Nx % 2 == 0);
         // stage X_k (k = 0..M) in bufB (zero padding, Nyquist plane and Im(DC) removed)
         const int nX = even ? M + 1 : Nxp / 2 + 1;
         for (int idx = tid; idx < LPB * nX; idx += XNT) {
             int ln = idx / nX, k = idx - ln * nX;
             long long gl = gl0 + ln;
             double2 v = czero();
-            if (gl < nlines && k < Nxh && !(xeven && k == a.gd.Nx / 2)) {
-                v = in[(size_t)gl * Nxh + k];
-                if (sub) v = x_minus_i(v, sub[(size_t)gl * Nxh + k], a.gd.alpha * k);
+            if (gl < nlines && k < a.gd.nk) {
+                v = in[(size_t)gl * a.gd.ldk + k];
+                if (sub) v = x_minus_i(v, sub[(size_t)gl * a.gd.ldk + k], a.gd.alpha * k);
             }
             if (k == 0) v.y = 0.0;
             if (even && k == M) v.y = 0.0;
@@ -278,8 +277,9 @@ struct XCtx {
         }
         __syncthreads();
         double2* res = lds_fft(bufA, bufB, a.plan, LPB, ld, -1, tid, XNT);
-        for (int idx = tid; idx < LPB * Nxh; idx += XNT) {
-            int ln = idx / Nxh, k = idx - ln * Nxh;
+        const int nk = a.gd.nk;
+        for (int idx = tid; idx < LPB * nk; idx += XNT) {
+            int ln = idx / nk, k = idx - ln * nk;
             long long gl = gl0 + ln;
             if (gl >= nlines) continue;
             double2 X;
@@ -288,7 +288,7 @@ struct XCtx {
             } else {
                 X = res[ln * ld + k];
             }
-            out[(size_t)gl * Nxh + k] = X;
+            out[(size_t)gl * a.gd.ldk + k] = X;
         }
         __syncthreads();
     }
@@ -323,8 +323,7 @@ __host__ __device__ constexpr int x_region_slots(int mode, int ppt, int ld) { re
 template <typename C>
 __device__ __forceinline__ C x_coef(const XArgs& a, int f, long long gl, int k, int M) {
     C v = cplx<C>(0, 0);
-    if (k < a.gd.Nxh && !((a.gd.Nx % 2 == 0) && k == a.gd.Nx / 2))
-        v = reinterpret_cast<const C*>(a.in[f])[(size_t)gl * a.gd.Nxh + k];
+    if (k < a.gd.nk) v = reinterpret_cast<const C*>(a.in[f])[(size_t)gl * a.gd.ldk + k];
     if (k == 0 || k == M) v.y = 0;
     return v;
 }
@@ -346,9 +345,8 @@ __device__ __forceinline__ void xpass_wave(const XArgs& a, C* smem, unsigned blo
     using T = creal_t<C>;
     constexpr int NIN = x_fields_in(MODE), NFFT = x_fft_lines_in(MODE), NOUT = x_fields_out(MODE);
     constexpr int NB = x_buffer_lines(MODE);
-    const int Nxp = a.gd.Nxp, Nxh = a.gd.Nxh, M = Nxp / 2, ld = a.ld;
+    const int Nxp = a.gd.Nxp, nk = a.gd.nk, ldk = a.gd.ldk, M = Nxp / 2, ld = a.ld;
     const long long nlines = (long long)a.gd.Nzp * a.gd.Ny;
-    const bool xeven = (a.gd.Nx % 2 == 0);
     // twiddles: FFT table (M) and pack/unpack table exp(-2 pi i k / Nxp), k <= M
     C* tw = smem;
     C* twx = smem + M;
@@ -417,9 +415,9 @@ __device__ __forceinline__ void xpass_wave(const XArgs& a, C* smem, unsigned blo
         }
         wave_sync();
         lds_fft_inplace<PPT, true>(bufA, a.plan, (const C*)tw, 3, ld, -1, lane, 64);
-        for (int idx = lane; idx < 3 * Nxh; idx += 64) {
-            const int c = (int)fast_div((unsigned)idx, a.mul_nxh), k = idx - c * Nxh;
-            reinterpret_cast<C*>(a.out[c])[(size_t)gl * Nxh + k] =
+        for (int idx = lane; idx < 3 * nk; idx += 64) {
+            const int c = (int)fast_div((unsigned)idx, a.mul_nk), k = idx - c * nk;
+            reinterpret_cast<C*>(a.out[c])[(size_t)gl * ldk + k] =
                 x_unpack(bufA[c * ld + k], bufA[c * ld + ((M - k) % M)], twx[k]);
         }
         return;
@@ -429,10 +427,10 @@ __device__ __forceinline__ void xpass_wave(const XArgs& a, C* smem, unsigned blo
         // lines (global_load_lds: no registers, every load in flight at
         // once); padding k = Nxh..M and the x Nyquist k = Nx/2 are zero.
         static_assert(sizeof(C) == 16, "direct LDS loads move 16-byte elements");
-        const int nload = xeven ? a.gd.Nx / 2 : Nxh;  // retained coefficients, Nyquist excluded
+        const int nload = nk;  // retained coefficients, Nyquist excluded
 #pragma unroll
         for (int f = 0; f < 6; ++f) {
-            const C* src = reinterpret_cast<const C*>(a.in[f]) + (size_t)gl * Nxh;
+            const C* src = reinterpret_cast<const C*>(a.in[f]) + (size_t)gl * ldk;
             for (int k0 = 0; k0 < nload; k0 += 64)
                 if (k0 + lane < nload)
                     __builtin_amdgcn_global_load_lds((const void*)(src + k0 + lane),
@@ -551,9 +549,9 @@ __device__ __forceinline__ void xpass_wave(const XArgs& a, C* smem, unsigned blo
         }
         wave_sync();
         lds_fft_inplace<PPT, true>(bufA, a.plan, (const C*)tw, NOUT, ld, -1, lane, 64);
-        for (int idx = lane; idx < NOUT * Nxh; idx += 64) {
-            int c = (int)fast_div((unsigned)idx, a.mul_nxh), k = idx - c * Nxh;
-            reinterpret_cast<C*>(a.out[c])[(size_t)gl * Nxh + k] =
+        for (int idx = lane; idx < NOUT * nk; idx += 64) {
+            int c = (int)fast_div((unsigned)idx, a.mul_nk), k = idx - c * nk;
+            reinterpret_cast<C*>(a.out[c])[(size_t)gl * ldk + k] =
                 x_unpack(bufA[c * ld + k], bufA[c * ld + ((M - k) % M)], twx[k]);
         }
         return;
@@ -564,10 +562,10 @@ __device__ __forceinline__ void xpass_wave(const XArgs& a, C* smem, unsigned blo
     for (int idx = lane; idx < NIN * nX; idx += 64) {
         int f = (int)fast_div((unsigned)idx, a.mul_nx), k = idx - f * nX;
         C v = cplx<C>(0, 0);
-        if (k < Nxh && !(xeven && k == a.gd.Nx / 2)) {
-            v = reinterpret_cast<const C*>(a.in[f])[(size_t)gl * Nxh + k];
+        if (k < nk) {
+            v = reinterpret_cast<const C*>(a.in[f])[(size_t)gl * ldk + k];
             if constexpr (MODE == X_ROTATIONAL)  // Omega_y = field 4 - i alpha k V_z
-                if (f == 4) v = x_minus_i(v, reinterpret_cast<const C*>(a.in[2])[(size_t)gl * Nxh + k], T(a.gd.alpha * k));
+                if (f == 4) v = x_minus_i(v, reinterpret_cast<const C*>(a.in[2])[(size_t)gl * ldk + k], T(a.gd.alpha * k));
         }
         if (k == 0 || k == M) v.y = 0;
         bufB[f * ld + k] = v;
@@ -628,9 +626,9 @@ __device__ __forceinline__ void xpass_wave(const XArgs& a, C* smem, unsigned blo
     }
     wave_sync();
     C* r2 = lds_fft<true>(nxt, res, a.plan, (const C*)tw, NOUT, ld, -1, lane, 64);
-    for (int idx = lane; idx < NOUT * Nxh; idx += 64) {
-        int c = (int)fast_div((unsigned)idx, a.mul_nxh), k = idx - c * Nxh;
-        reinterpret_cast<C*>(a.out[c])[(size_t)gl * Nxh + k] = x_unpack(r2[c * ld + k], r2[c * ld + ((M - k) % M)], twx[k]);
+    for (int idx = lane; idx < NOUT * nk; idx += 64) {
+        int c = (int)fast_div((unsigned)idx, a.mul_nk), k = idx - c * nk;
+        reinterpret_cast<C*>(a.out[c])[(size_t)gl * ldk + k] = x_unpack(r2[c * ld + k], r2[c * ld + ((M - k) % M)], twx[k]);
     }
 }
 
@@ -747,9 +745,10 @@ static void launch_z(const ZArgs& a, dim3 grid, size_t lds, hipStream_t st) {
 }
 
 hipError_t launch_zpass(int dir, const ZArgs& a, hipStream_t st) {
+    if (a.r1 > 0) return launch_zreg(dir, a, st);
     if (a.ppt != 0 && a.ppt != 8 && a.ppt != 16) return hipErrorInvalidValue;
     if (a.mixed && a.ppt == 0) return hipErrorInvalidValue;  // FP32 fields: in-place plans only
-    dim3 grid((unsigned)((a.gd.Nxh + a.KT - 1) / a.KT) * (unsigned)a.gd.Ny * (unsigned)a.nfields);
+    dim3 grid((unsigned)((a.gd.nk + a.KT - 1) / a.KT) * (unsigned)a.gd.Ny * (unsigned)a.nfields);
     size_t lds = z_lds_bytes(a);
     if (dir > 0) launch_z<+1>(a, grid, lds, st);
     else launch_z<-1>(a, grid, lds, st);
@@ -757,7 +756,7 @@ hipError_t launch_zpass(int dir, const ZArgs& a, hipStream_t st) {
 }
 
 unsigned z_blocks(const ZArgs& a) {
-    return (unsigned)((a.gd.Nxh + a.KT - 1) / a.KT) * (unsigned)a.gd.Ny * (unsigned)a.nfields;
+    return (unsigned)((a.gd.nk + a.KT - 1) / a.KT) * (unsigned)a.gd.Ny * (unsigned)a.nfields;
 }
 
 hipError_t launch_zpass_batch(int dir, int ppt, const ZArgs* tab, const unsigned* start, int n, unsigned nblocks,

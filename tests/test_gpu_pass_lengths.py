@@ -1,0 +1,32 @@
+"""Periodic passes at the edges of their length rules: lines kept in one lane,
+each pair of register radices, lengths with no such pair (the staged passes),
+widths that do not divide the tile.  Transforms against the oracle, at the flat
+1e-13 that every transform of the repository is held to; the nonlinear step
+against the oracle's step within its roundoff envelope."""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+from test_gpu_parity import hermitian_random, make, rel, say
+
+pytestmark = pytest.mark.gpu
+
+# padded z lengths 2, 3, 11, 12, 14, 21, 24, 48, 50, 98, 105, 192, 225, 288, 360, 384, 432, 504, 576, 600
+NZ = [1, 2, 7, 8, 9, 14, 16, 32, 33, 65, 70, 128, 150, 192, 240, 256, 288, 336, 384, 400]
+
+
+@pytest.mark.parametrize("Nz", NZ)
+@pytest.mark.parametrize("Nx", [5, 12, 34])
+def test_z_lengths(gpu, Nz, Nx):
+    import torch
+    cf = gpu
+    say("z length", Nx, Nz)
+    gc, go, prob = make(cf, (Nx, 5, Nz))
+    rng = np.random.default_rng(Nz + 1000 * Nx)
+    u = rng.standard_normal((3,) + go.phys_shape)
+    F = cf.FFT(prob, torch.as_tensor(u, device="cuda")).cpu().numpy()
+    U = hermitian_random(go, rng, 3)
+    v = cf.IFFT(prob, torch.as_tensor(U, device="cuda")).cpu().numpy()
+    for c in range(3):
+        assert rel(F[c], O.forward(go, u[c])) < 1e-13
+        assert rel(v[c], O.inverse(go, U[c])) < 1e-13
