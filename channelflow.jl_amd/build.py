@@ -18,8 +18,8 @@ LIB = os.path.join(LIBDIR, "libcfhip.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
 # heaviest translation units first (the wall-normal layouts, then the x/z passes)
-SOURCES = [*[f"kernels_y_p{p}.hip" for p in (6, 7, 4, 3, 2, 1, 5)], "kernels_xz.hip", "kernels_zreg.hip", "kernels_closure.hip", "kernels_y.hip",
-           "kernels_rng.hip", "scratch.hip", "setup.cpp", "api.cpp"]
+SOURCES = [*[f"kernels_y_p{p}.hip" for p in (6, 7, 4, 3, 2, 1, 5)], *[f"kernels_xreg_p{p}.hip" for p in (3, 4, 1, 2, 6, 7, 5)],
+           "kernels_xreg.hip", "kernels_xz.hip", "kernels_zreg.hip", "kernels_closure.hip", "kernels_y.hip", "kernels_rng.hip", "scratch.hip", "setup.cpp", "api.cpp"]
 
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",

@@ -94,6 +94,7 @@ struct cf_problem {
     int xwaves = 4;  // even Nxp: wavefronts per block of the nonlinear x pass
     int zppt = 0;    // z pass in-place points per thread (0: two buffers)
     int zr1 = 0, zr2 = 0;  // register radices of the FP64 z pass (0: none, the staged passes)
+    int xr1 = 0, xr2 = 0;  // the same of the FP64 x pass
     int xppt = 0;    // even-Nxp x pass in-place points per lane (0: two buffers)
     // forcing(tstage, U, F) hook: host callback and the caller's F fields
     cf_forcing_fn force_fn = nullptr;
@@ -403,6 +404,7 @@ extern "C" int cf_problem_create(const cf_config* cfg, cf_problem** out) {
     if ((rc = make_plan(h, gd.Nzp, h->pz))) return bail(rc);
     if ((rc = make_plan(h, 2 * gd.P, h->py))) return bail(rc);
     (void)z_reg_split(gd.Nzp, &h->zr1, &h->zr2);
+    (void)x_reg_split(gd.Nxp, &h->xr1, &h->xr2);
     int M = (gd.Nxp % 2 == 0) ? gd.Nxp / 2 : gd.Nxp;
     if ((rc = make_plan(h, M, h->px))) return bail(rc);
     {
@@ -588,6 +590,16 @@ static ZArgs make_zargs(cf_problem* h, int nf, double2* const* in, double2* cons
     return z;
 }
 
+// the register x pass of x.mode where the padded length splits (r1 = 0: the
+// staged passes stand)
+static void x_registers(cf_problem* h, XArgs& x) {
+    if (!h->xr1) return;
+    x.r1 = h->xr1;
+    x.r2 = h->xr2;
+    if (x.mode == X_ROT_SPLIT || x.mode == X_ROT_ASYNC) x.mode = X_ROTATIONAL;
+    x_reg_shape(x);
+}
+
 static int zpass(cf_problem* h, int dir, int nf, double2* const* in, double2* const* out, hipStream_t st,
                  unsigned dz_mask = 0, bool mixed = false) {
     HIPTRY(launch_zpass(dir, make_zargs(h, nf, in, out, dz_mask, mixed), st));
@@ -630,7 +642,7 @@ struct NonlinearArgs {
     XArgs x;
 };
 
-// staged: the z passes of the setup calls (cf_nonlinear, cf_pressure) keep the
+// staged: the passes of the setup calls (cf_nonlinear, cf_pressure) keep the
 // staged multi-pass transforms.  An FP32-mixed run amplifies a last-bit change
 // of its initial pressure to FP32 noise within one step, so the calls that
 // prepare it keep their bits; they run once per trajectory.
@@ -677,6 +689,8 @@ static NonlinearArgs nonlinear_args(cf_problem* h, bool mixed, bool staged = fal
     na.zout = make_zargs(h, nout, zb, six, 0, mixed);
     if (staged)
         for (ZArgs* z : {&na.zin, &na.zout}) z->r1 = z->r2 = 0;
+    else if (!mixed)
+        x_registers(h, x);
     return na;
 }
 
@@ -1061,6 +1075,7 @@ static int velocity_gradient_on(cf_problem* h, double2* const U[3], double* out,
         x.in[i] = zb[i];
         x.rout[i] = out + nphys * i;
     }
+    x_registers(h, x);
     HIPTRY(launch_xpass(x, st));
     return CF_OK;
 }
@@ -1316,6 +1331,7 @@ static int forward_fields(cf_problem* h, int nf, const double* u, double* const*
         a.Nphys[c] = zo[c];
         a.Rout[c] = (double2*)U[c];
     }
+    x_registers(h, x);
     HIPTRY(launch_xpass(x, st));
     if (int rc = zpass(h, -1, nf, zi, zo, st)) return rc;
     HIPTRY(launch_ykernel(Y_DCT_FWD, a, st));
@@ -1342,6 +1358,7 @@ static int inverse_fields(cf_problem* h, int nf, double* const* U, double* u, hi
     }
     HIPTRY(launch_ykernel(Y_DCT_INV, a, st));
     if (int rc = zpass(h, +1, nf, zi, zo, st)) return rc;
+    x_registers(h, x);
     HIPTRY(launch_xpass(x, st));
     return CF_OK;
 }
@@ -1698,7 +1715,7 @@ extern "C" int cf_problem_tune(cf_problem* h, void* stream) {
     h->zppt = bestPPT;
     // x pass: wavefronts per block (even padded Nx), and for the rotating
     // form the six-line or the split (three-line) variant
-    if (!rc && h->gd.Nxp % 2 == 0) {
+    if (!rc && h->gd.Nxp % 2 == 0 && !h->xr1) {
         const int keepSplit = h->xsplit;
         int bestW[3] = {h->xwaves, h->xwavess, h->xwavesa}, bestSplit = keepSplit;
         int* waves[3] = {&h->xwaves, &h->xwavess, &h->xwavesa};
@@ -1876,6 +1893,7 @@ extern "C" int cf_problem_set_tiles(cf_problem* h, const int tiles[5]) {
 namespace {
 
 enum { B_YPRO = 0, B_ZINV, B_X, B_ZFWD, B_YSTAGE };
+constexpr int XR_KEY = 64;  // register x pass: mode + XR_KEY * (largest radix of its class)
 
 struct BatchLaunch {
     int cls;        // B_*
@@ -1928,7 +1946,10 @@ static hipError_t run_batch(const BatchLaunch& b, hipStream_t st) {
             if (b.waves) return launch_zreg_batch(dir, b.tp, 64 * b.waves, (const ZArgs*)b.tab, b.start, b.n, b.nblocks, b.lds, st);
             return launch_zpass_batch(dir, b.tp, (const ZArgs*)b.tab, b.start, b.n, b.nblocks, b.lds, st);
         }
-        case B_X: return launch_xpass_batch(b.mode, b.tp, b.waves, (const XArgs*)b.tab, b.start, b.n, b.nblocks, b.lds, st);
+        case B_X:
+            if (b.mode >= XR_KEY)
+                return launch_xreg_batch(b.mode % XR_KEY, b.tp, b.mode / XR_KEY, b.waves, (const XArgs*)b.tab, b.start, b.n, b.nblocks, b.lds, st);
+            return launch_xpass_batch(b.mode, b.tp, b.waves, (const XArgs*)b.tab, b.start, b.n, b.nblocks, b.lds, st);
         default: return hipErrorInvalidValue;
     }
 }
@@ -2006,7 +2027,7 @@ static int ens_build(cf_ensemble* e, std::vector<BatchLaunch>& step) {
             z->ppt = t.zppt;
             z->mul_kt = recip_mul((unsigned)t.KT);
         }
-        na.x.waves = t.xwaves;
+        if (!na.x.r1) na.x.waves = t.xwaves;
         zin[i] = na.zin;
         zout[i] = na.zout;
         xs[i] = na.x;
@@ -2026,10 +2047,13 @@ static int ens_build(cf_ensemble* e, std::vector<BatchLaunch>& step) {
         b = z_blocks(a);
         l = a.r1 ? z_reg_lds(a) : z_lds_bytes(a);
     };
-    auto xkey = [](const XArgs& a) { return std::array<int, 3>{a.ppt, a.waves, a.mode}; };
+    auto xkey = [](const XArgs& a) {
+        return a.r1 ? std::array<int, 3>{a.r2, a.waves, a.mode + XR_KEY * (a.r1 <= 12 ? 12 : 24)}
+                    : std::array<int, 3>{a.ppt, a.waves, a.mode};
+    };
     auto xinfo = [](const XArgs& a, unsigned& b, size_t& l) {
-        b = x_blocks(a);
-        l = x_lds_bytes(a);
+        b = a.r1 ? x_reg_blocks(a) : x_blocks(a);
+        l = a.r1 ? x_reg_lds(a) : x_lds_bytes(a);
     };
     step.clear();
     if (int rc = ens_class(e, B_YPRO, pro, ykey, yinfo, step)) return rc;
@@ -2110,7 +2134,7 @@ static int ens_tune(cf_ensemble* e) {
         // x wavefronts per block (LDS permitting)
         best = 1e30f;
         int wkeep = e->tiles[members[0]].xwaves;
-        for (int w = 1; w <= h->xmaxw[0]; w *= 2) {
+        for (int w = 1; w <= h->xmaxw[0] && !h->xr1; w *= 2) {
             for (int i : members) e->tiles[i].xwaves = w;
             float ms;
             if (int rc = ens_time_class(e, B_X, &ms)) return rc;

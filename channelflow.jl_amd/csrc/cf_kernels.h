@@ -105,6 +105,11 @@ struct XArgs {
     int ppt;               // even Nxp: in-place FFT points per lane (one LDS buffer), 0: two buffers
     unsigned long long mul_m, mul_nk, mul_nx;  // recip_mul of Nxp/2, nk and Nxp/2+1 (index splits)
     int mixed;             // 1: in/out are FP32 complex (float2); even Nxp, in-place wave path only
+    // r1 > 0: register radices, Nxp = r1 r2 (x_reg_split; FP64), nl lines in a
+    // block of `waves` wavefronts; workspace fields Sz and physical fields
+    // Nxp Nzp Ny apart
+    int r1, r2, nl;
+    unsigned long long mul_nl, mul_r1;
     const double2* in[9];  // (k, zp, y) complex, nk per line of ldk
     double2* out[6];
     const double* rin[3];  // (x, zp, y) real
@@ -181,6 +186,13 @@ size_t z_reg_lds(const ZArgs& a);
 hipError_t launch_zreg_batch(int dir, int cls, int nthreads, const ZArgs* tab, const unsigned* start, int n,
                              unsigned nblocks, size_t lds, hipStream_t st);
 hipError_t launch_xpass(const XArgs& a, hipStream_t st);
+bool x_reg_split(int n, int* r1, int* r2);  // false: n = r1 r2 has no such split
+void x_reg_shape(XArgs& a);                 // nl, waves and reciprocals of a.r1, a.r2 for the form
+size_t x_reg_lds(const XArgs& a);
+unsigned x_reg_blocks(const XArgs& a);
+hipError_t launch_xreg(const XArgs& a, hipStream_t st);
+hipError_t launch_xreg_batch(int mode, int r2, int rmax, int waves, const XArgs* tab, const unsigned* start, int n,
+                             unsigned nblocks, size_t lds, hipStream_t st);
 size_t x_lds_bytes(const XArgs& a);
 int x_phys_lines(int mode);  // physical lines per (zp, y) line of the odd-Nxp x pass
 int x_max_waves(const XArgs& a);  // even Nxp: wavefronts per block that fit the LDS (0: none)

@@ -859,6 +859,7 @@ hipError_t launch_xpass_batch(int mode, int ppt, int waves, const XArgs* tab, co
 }
 
 hipError_t launch_xpass(const XArgs& a, hipStream_t st) {
+    if (a.r1 > 0) return launch_xreg(a, st);
     long long nlines = (long long)a.gd.Nzp * a.gd.Ny;
     const bool wave = x_wave_path(a);
     if (wave && (a.waves < 1 || a.waves > XNT / 64)) return hipErrorInvalidValue;

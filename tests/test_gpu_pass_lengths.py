@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 
 from oracle import oracle as O
-from test_gpu_parity import hermitian_random, make, rel, say
+from test_gpu_parity import _split, assert_parity, hermitian_random, make, rel, run_pair, say
 
 pytestmark = pytest.mark.gpu
 
@@ -30,3 +30,32 @@ def test_z_lengths(gpu, Nz, Nx):
     for c in range(3):
         assert rel(F[c], O.forward(go, u[c])) < 1e-13
         assert rel(v[c], O.inverse(go, U[c])) < 1e-13
+
+
+# padded x lengths 2, 3, 5, 6, 8, 9, 11, 12, 14, 21, 33 and 51 (odd, 51 staged), 63, 81, 98 .. 384: each register
+# class of the x pass, the shortest lines, odd and even, and lengths that keep the staged pass
+NX = [1, 2, 3, 4, 5, 6, 7, 8, 9, 14, 22, 34, 42, 54, 65, 70, 96, 128, 150, 160, 192, 200, 256, 300]
+
+
+@pytest.mark.parametrize("Nx", NX)
+def test_x_lengths(gpu, Nx):
+    import torch
+    cf = gpu
+    say("x length", Nx)
+    gc, go, prob = make(cf, (Nx, 5, 6))
+    rng = np.random.default_rng(Nx)
+    u = rng.standard_normal((3,) + go.phys_shape)
+    F = cf.FFT(prob, torch.as_tensor(u, device="cuda")).cpu().numpy()
+    U = hermitian_random(go, rng, 3)
+    v = cf.IFFT(prob, torch.as_tensor(U, device="cuda")).cpu().numpy()
+    for c in range(3):
+        assert rel(F[c], O.forward(go, u[c])) < 1e-13
+        assert rel(v[c], O.inverse(go, U[c])) < 1e-13
+
+
+@pytest.mark.parametrize("form", ["rotating", "convective", "divergence"])
+@pytest.mark.parametrize("Nx", [3, 4, 5, 8, 14, 30, 42, 64, 65, 100, 150, 200, 256])
+def test_x_lengths_step(gpu, Nx, form):
+    say("x length step", form, Nx)
+    U, P, Ur, Pr, _, _, env = run_pair(gpu, (Nx, 9, 6), 1, form=form)
+    assert_parity(f"step {form} {Nx}", _split((U, P)), _split((Ur, Pr)), env)
