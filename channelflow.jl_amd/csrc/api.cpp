@@ -726,8 +726,11 @@ static YArgs prologue_args(cf_problem* h, double2* const U[3], bool mixed) {
     return a;
 }
 
-static int enqueue_prologue(cf_problem* h, double2* const U[3], hipStream_t st, bool mixed = false) {
-    HIPTRY(launch_ykernel(Y_PROLOGUE, prologue_args(h, U, mixed), st));
+// staged: as for enqueue_nonlinear_phys
+static int enqueue_prologue(cf_problem* h, double2* const U[3], hipStream_t st, bool mixed = false, bool staged = false) {
+    YArgs a = prologue_args(h, U, mixed);
+    if (staged) a.r1 = -1;
+    HIPTRY(launch_ykernel(Y_PROLOGUE, a, st));
     return 0;
 }
 
@@ -1397,7 +1400,7 @@ extern "C" int cf_inverse3(cf_problem* h, const double* U0, const double* U1, co
 
 // nonlinear term of U into spectral N (3 fields)
 static int enqueue_nonlinear_spec(cf_problem* h, double2* const U[3], double2* const N[3], hipStream_t st) {
-    if (int rc = enqueue_prologue(h, U, st)) return rc;
+    if (int rc = enqueue_prologue(h, U, st, false, true)) return rc;
     if (int rc = enqueue_nonlinear_phys(h, st, nullptr, false, true)) return rc;
     if (h->form == CF_FORM_DIVERGENCE) return enqueue_nonlinear_coef(h, N, st);
     YArgs a = base_yargs(h);
@@ -1938,8 +1941,8 @@ static void ens_free(cf_ensemble* e) {
 
 static hipError_t run_batch(const BatchLaunch& b, hipStream_t st) {
     switch (b.cls) {
-        case B_YPRO: return launch_ykernel_batch(Y_PROLOGUE, b.tp, (const YArgs*)b.tab, b.start, b.n, b.nblocks, b.lds, st);
-        case B_YSTAGE: return launch_ykernel_batch(Y_STAGE, b.tp, (const YArgs*)b.tab, b.start, b.n, b.nblocks, b.lds, st);
+        case B_YPRO: return launch_ykernel_batch(Y_PROLOGUE, b.tp, b.waves, (const YArgs*)b.tab, b.start, b.n, b.nblocks, b.lds, st);
+        case B_YSTAGE: return launch_ykernel_batch(Y_STAGE, b.tp, b.waves, (const YArgs*)b.tab, b.start, b.n, b.nblocks, b.lds, st);
         case B_ZINV:
         case B_ZFWD: {
             const int dir = b.cls == B_ZINV ? +1 : -1;
@@ -2020,6 +2023,7 @@ static int ens_build(cf_ensemble* e, std::vector<BatchLaunch>& step) {
         Constraint c;
         if (int rc = resolve_constraint(h, -1, nullptr, c)) return rc;
         pro[i] = prologue_args(h, U, false);
+        y_reg_split(pro[i], y_group_lanes(h->gd.Ny), y_group_k(h->gd.Ny));
         NonlinearArgs na = nonlinear_args(h, false);
         const Tiles& t = e->tiles[i];
         for (ZArgs* z : {&na.zin, &na.zout}) {
@@ -2032,12 +2036,15 @@ static int ens_build(cf_ensemble* e, std::vector<BatchLaunch>& step) {
         zout[i] = na.zout;
         xs[i] = na.x;
         double2* Nc[3] = {nullptr, nullptr, nullptr};
-        for (int j = 0; j < 3; ++j) stages[i][j] = stage_args(h, U, e->fields[i][3], j, c, h->dt, &h->stage[j], false, Nc);
+        for (int j = 0; j < 3; ++j) {
+            stages[i][j] = stage_args(h, U, e->fields[i][3], j, c, h->dt, &h->stage[j], false, Nc);
+            y_reg_split(stages[i][j], y_group_lanes(h->gd.Ny), y_group_k(h->gd.Ny));
+        }
     }
-    auto ykey = [](const YArgs& a) { return std::array<int, 3>{y_group_lanes(a.gd.Ny), 0, 0}; };
+    auto ykey = [](const YArgs& a) { return std::array<int, 3>{y_group_lanes(a.gd.Ny), a.r1 > 0, 0}; };
     auto yinfo = [](const YArgs& a, unsigned& b, size_t& l) {
         b = y_blocks(a.gd);
-        l = y_lds_bytes(a.gd.Ny, a.ld);
+        l = a.r1 ? y_reg_lds(a, y_group_lanes(a.gd.Ny), 4) : y_lds_bytes(a.gd.Ny, a.ld);
     };
     // register z passes: one launch per register class and block size
     auto zkey = [](const ZArgs& a) {

@@ -73,6 +73,9 @@ struct YArgs {
     // Y_STAGE / Y_PROLOGUE: group layout, L lanes of K coefficients per mode
     // (yk = 0: the default layout of Ny; other kernels always use it)
     int yl, yk;
+    // r1 > 0: register radices of the DCT, 2P = r1 r2 (y_reg_split), nf fields
+    // a pass, zs LDS slots a line; r1 = -1 asks for the staged transforms
+    int r1, r2, nf, zs;
 };
 
 struct ZArgs {
@@ -174,6 +177,10 @@ int y_group_k(int Ny);      // coefficients K per lane (4; 6 above 256 points, 8
 // not cover Ny coefficients
 size_t y_lds_bytes_layout(int Ny, int ld, int L, int K);
 size_t y_lds_bytes(int Ny, int ld);
+// register radices of a Y_STAGE / Y_PROLOGUE launch in layout (L, K) into
+// a.r1 .. a.zs (a.r1 = 0: the length has none)
+void y_reg_split(YArgs& a, int L, int K);
+size_t y_reg_lds(const YArgs& a, int L, int K);  // LDS bytes of that launch
 hipError_t launch_zpass(int dir, const ZArgs& a, hipStream_t st);
 size_t z_lds_bytes(const ZArgs& a);
 int z_inplace_ppt(const FFTPlan& plan, int KT);  // 0: the plan needs two buffers
@@ -202,7 +209,7 @@ int x_inplace_ppt(const XArgs& a);  // even Nxp: in-place points per lane for th
 // [start[i], start[i+1]) of an nblocks grid and reads its arguments from
 // tab[i] (device memory).  All instances of one launch share the template
 // parameters named in the call; lds is the largest instance's need.
-hipError_t launch_ykernel_batch(int which, int L, const YArgs* tab, const unsigned* start, int n, unsigned nblocks,
+hipError_t launch_ykernel_batch(int which, int L, bool reg, const YArgs* tab, const unsigned* start, int n, unsigned nblocks,
                                 size_t lds, hipStream_t st);  // Y_STAGE or Y_PROLOGUE
 hipError_t launch_zpass_batch(int dir, int ppt, const ZArgs* tab, const unsigned* start, int n, unsigned nblocks,
                               size_t lds, hipStream_t st);

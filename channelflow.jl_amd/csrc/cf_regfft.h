@@ -113,6 +113,22 @@ template <> struct RegTwiddle<24> {
         -0.9659258262890683, -1.0, -0.9659258262890683, -0.8660254037844386, -0.7071067811865476, -0.5,
         -0.25881904510252074};
 };
+template <> struct RegTwiddle<32> {
+    static constexpr double c[32] = {1.0, 0.9807852804032304, 0.9238795325112867, 0.8314696123025452,
+        0.7071067811865476, 0.5555702330196022, 0.3826834323650898, 0.19509032201612828, 0.0,
+        -0.19509032201612828, -0.3826834323650898, -0.5555702330196022, -0.7071067811865476,
+        -0.8314696123025452, -0.9238795325112867, -0.9807852804032304, -1.0, -0.9807852804032304,
+        -0.9238795325112867, -0.8314696123025452, -0.7071067811865476, -0.5555702330196022, -0.3826834323650898,
+        -0.19509032201612828, 0.0, 0.19509032201612828, 0.3826834323650898, 0.5555702330196022,
+        0.7071067811865476, 0.8314696123025452, 0.9238795325112867, 0.9807852804032304};
+    static constexpr double s[32] = {0.0, 0.19509032201612828, 0.3826834323650898, 0.5555702330196022,
+        0.7071067811865476, 0.8314696123025452, 0.9238795325112867, 0.9807852804032304, 1.0, 0.9807852804032304,
+        0.9238795325112867, 0.8314696123025452, 0.7071067811865476, 0.5555702330196022, 0.3826834323650898,
+        0.19509032201612828, 0.0, -0.19509032201612828, -0.3826834323650898, -0.5555702330196022,
+        -0.7071067811865476, -0.8314696123025452, -0.9238795325112867, -0.9807852804032304, -1.0,
+        -0.9807852804032304, -0.9238795325112867, -0.8314696123025452, -0.7071067811865476, -0.5555702330196022,
+        -0.3826834323650898, -0.19509032201612828};
+};
 
 // R = A B; primes and 4, 8 are written out
 template <int R> struct RegSplit { static constexpr int A = 0, B = 0; };
@@ -127,6 +143,7 @@ template <> struct RegSplit<18> { static constexpr int A = 6, B = 3; };
 template <> struct RegSplit<20> { static constexpr int A = 4, B = 5; };
 template <> struct RegSplit<21> { static constexpr int A = 3, B = 7; };
 template <> struct RegSplit<24> { static constexpr int A = 8, B = 3; };
+template <> struct RegSplit<32> { static constexpr int A = 8, B = 4; };
 
 __device__ __forceinline__ double2 rot90(double2 a, int dir) { return dir < 0 ? cmulni(a) : cmuli(a); }  // a * exp(dir i pi/2)
 

@@ -11,8 +11,11 @@
 // (src/solvers/stokes.jl:81-108, batchedinfluence.jl:129-159, meanmode.jl:103-150),
 // Chebyshev transforms (src/ffts.jl:65-82,151-166, transforms/chebyshev.jl:45-66),
 // curl (src/fields/operators.jl:172-190), pressure (src/pressure.jl:196-285).
+#include <type_traits>
+
 #include "cf_device.h"
 #include "cf_kernels.h"
+#include "cf_regfft.h"
 
 // This file is compiled as several translation units so that the layouts
 // build in parallel: part 0 (this file on its own) holds the dispatchers and
@@ -49,6 +52,36 @@ __device__ __forceinline__ ModeInfo mode_info(const GridDims& gd, long long s) {
     return mi;
 }
 
+// Radices of the register DCT (Tile::dct_*_reg) built for a layout: those that
+// split the lengths 2P its Ny range holds, as few as cover the 7-smooth P (the
+// largest one sets the kernel's registers).  The layouts without any (K = 8,
+// and K = 6 on 32 lanes) keep the staged transforms.
+__host__ __device__ constexpr bool y_radix(int L, int K, int r) {
+    if (K == 6) return L == 64 && (r == 16 || r == 18 || r == 20 || r == 21 || r == 24 || r == 32);
+    if (K != 4) return false;
+    if (L == 4) return r >= 2 && r <= 7;
+    if (L == 8) return r >= 3 && r <= 10;
+    if (L == 16) return (r >= 6 && r <= 10) || r == 12 || r == 14;
+    if (L == 32) return (r >= 8 && r <= 10) || r == 12 || (r >= 14 && r <= 16) || r == 18 || r == 20;
+    return r == 12 || (r >= 14 && r <= 16) || r == 18 || r == 20 || r == 21 || r == 24;
+}
+template <int L, int K>
+constexpr bool y_has_reg() { return K == 4 || (K == 6 && L == 64); }
+
+// f(radix r as a compile-time constant)
+template <int L, int K, int R = 2, typename F>
+__device__ __forceinline__ void with_radix(int r, F&& f) {
+    if constexpr (R <= 32) {
+        if constexpr (y_radix(L, K, R)) {
+            if (r == R) {
+                f(std::integral_constant<int, R>{});
+                return;
+            }
+        }
+        with_radix<L, K, R + 1>(r, f);
+    }
+}
+
 // LDS slots (double2) of the per-degree table: CHEB_TAB_ARRAYS arrays of K L doubles
 template <int L, int K>
 __host__ __device__ constexpr int y_table_slots() { return CHEB_TAB_ARRAYS * K * L / 2; }
@@ -68,7 +101,8 @@ struct Tile {
     const GridDims& gd;
     long long s, sw0;  // this group's mode, the wave's first mode
     int lane, mw, ld;
-    double2 *bufA, *bufB, *stash;
+    double2 *bufA, *bufB, *stash, *lines;  // lines: the block's regions as one
+    unsigned blk;                          // block index
     const double2* tw;
     // region: LDS slots per wave (y_region_slots); smem starts with the
     // twiddle table of the DCT plan (ntw entries) and the per-degree table
@@ -88,6 +122,8 @@ struct Tile {
         bufA = smem + ntw + y_table_slots<L, K>() + (size_t)wave * region;
         bufB = bufA + W * ld;
         stash = bufA + mw * 3 * K * L;
+        lines = smem + ntw + y_table_slots<L, K>();
+        blk = block;
     }
     // Non-Nyquist-first order (YOrder): the wave's first slot sw0 becomes a
     // mode index.  W divides nxr, so the wave's W slots lie in one z row and
@@ -113,6 +149,16 @@ struct Tile {
             int n = K * g.t + e;
             v.v[e] = (ok && n < gd.Ny) ? src[s + gd.B * n] : czero();
         }
+        return v;
+    }
+    // load of a column that this lane may have stored before (no forwarding of
+    // the stored registers: the index is opaque)
+    __device__ __forceinline__ CVec<K> reload(const double2* src, const Group<L, K>& g) const {
+        CVec<K> v;
+        long long i = s + gd.B * (K * g.t);
+        asm volatile("" : "+v"(i));
+#pragma unroll
+        for (int e = 0; e < K; ++e) v.v[e] = (s < gd.B && K * g.t + e < gd.Ny) ? src[i + gd.B * e] : czero();
         return v;
     }
     __device__ __forceinline__ void store(double2* __restrict__ dst, const Group<L, K>& g, const CVec<K>& v) const {
@@ -193,6 +239,197 @@ struct Tile {
         }
         wave_sync();
     }
+
+    // ---- DCT-I in two register radices, several fields a pass -------------
+    // The even extension has length N = 2P = r1 r2.  Its columns j + r2 r and
+    // (r2 - j) + r2 r mirror each other, and so do its output rows q + r1 p and
+    // (r1 - q) + r1 p: r2/2 + 1 columns and r1/2 + 1 rows are transformed, half
+    // of a length-2P transform.  First half: a lane holds one column of one
+    // mode and field, transforms it and leaves it twiddled in LDS, for its
+    // mirror column too (row pitch r2|1); second half: a lane gathers one row.
+    // One exchange through LDS instead of one per factor.  Bound by the issue of
+    // FP64 and LDS instructions beside the solves' scans; against the staged
+    // form, us a step: 32x33x32 186 -> 148, 64x65x64 282 -> 245, 128x97x128 824
+    // -> 787, 256x257x256 12550 -> 11865, 64-instance ensemble 1429 -> 1340.
+    // nf fields travel together so that the columns and rows fill the lanes: at
+    // Ny = 97 (12 x 16, two modes a wavefront) one field has 18 columns and 14
+    // rows, three have 54 and 42.
+    // SHARE: with one mode a wavefront (L = 64) the block's four modes share the
+    // work, neighbouring lanes holding neighbouring modes: 64 contiguous bytes a
+    // row where a wavefront on its own touches 16, and the address units bound
+    // it (256x257x256 step 12.37 -> 11.87 ms).  With two modes and more the
+    // block's barriers cost as much as that gains (32x33x32 step 148 us on
+    // wavefronts, 158 on blocks; 128x97x128 783 and 785).
+    static constexpr bool SHARE = L == 64;
+    static constexpr int RM = SHARE ? M : W;  // modes that share lines
+    static __device__ __forceinline__ void reg_sync() {
+        if constexpr (SHARE) __syncthreads();
+        else wave_sync();
+    }
+    struct RegItem {
+        int f, m, c;  // field within the pass, mode of the RM sharing lines, column or row
+        bool on;
+    };
+    __device__ __forceinline__ RegItem reg_item(int per, int nf) const {
+        // opaque to the optimiser: the addresses of every radix built would
+        // otherwise be hoisted out of the loop over the passes (registers)
+        int ln = SHARE ? (int)threadIdx.x : lane;
+        asm volatile("" : "+v"(ln));
+        const int rest = ln / RM;
+        RegItem it;
+        it.m = ln - rest * RM;
+        it.f = (rest >= per) + (rest >= 2 * per);
+        it.c = rest - it.f * per;
+        it.on = rest < per * nf;
+        return it;
+    }
+    // mode of slot m of those sharing lines (>= B: none)
+    __device__ __forceinline__ long long reg_mode(const YArgs& a, int m) const {
+        if constexpr (!SHARE) return sw0 + m;
+        const unsigned slot = blk * M + m;
+        if (!a.order.on) return slot;
+        if (slot >= (unsigned)a.order.nreg) return gd.B;
+        const unsigned q = slot / (unsigned)a.order.nxr;
+        return (long long)(q + (q >= (unsigned)a.order.zskip ? 1u : 0u)) * gd.Nxh + (slot - q * (unsigned)a.order.nxr);
+    }
+    __device__ __forceinline__ int line_slot() const { return SHARE ? (int)threadIdx.x / L : mw; }  // this group's m
+    __device__ __forceinline__ double2* reg_line(const YArgs& a, int f, int m) const {
+        return (SHARE ? lines : bufA) + (f * RM + m) * a.zs;
+    }
+    // twiddled column of R points -> LDS, and its mirror column
+    template <int R>
+    __device__ __forceinline__ void reg_column(const YArgs& a, const RegItem& it, double2* z, double2* v) const {
+        const int r2 = a.r2, pitch = r2 | 1, c = it.c, mc = r2 - c;
+        const bool mir = c > 0 && c != mc;
+        dft_reg<R>(v, -1);
+        if (!it.on) return;
+        z[c] = v[0];
+        if (mir) z[mc] = v[0];
+#pragma unroll
+        for (int q = 1; q <= R / 2; ++q) {
+            const double2 w = tw[c * q];
+            z[q * pitch + c] = cmul(v[q], w);
+            if (mir) z[q * pitch + mc] = cmul(v[R - q], cconj(w));
+        }
+    }
+    template <int R>
+    __device__ __forceinline__ void reg_row(const YArgs& a, const RegItem& it, const double2* z, double2* v) const {
+#pragma unroll
+        for (int j = 0; j < R; ++j) v[j] = it.on ? z[it.c * (a.r2 | 1) + j] : czero();
+        dft_reg<R>(v, -1);
+    }
+    // output p of row q: its degree, or -1 (a mirrored duplicate)
+    __device__ __forceinline__ int reg_out(const YArgs& a, const RegItem& it, int p) const {
+        const int k = it.c + a.r1 * p;
+        if (k <= gd.P) return it.on ? k : -1;
+        return (it.on && it.c != 0 && 2 * it.c != a.r1) ? 2 * gd.P - k : -1;
+    }
+    // three y-physical fields -> unscaled coefficients in the LDS lines
+    // reg_line(a, c, m) (row n at slot n)
+    template <typename SC>
+    __device__ __forceinline__ void dct_forward_reg(const YArgs& a, const SC* s0, const SC* s1, const SC* s2) {
+        const int P = gd.P, r1 = a.r1, r2 = a.r2, nf = a.nf;
+#pragma unroll 1
+        for (int base = 0; base < 3; base += nf) {
+            const int cnt = 3 - base < nf ? 3 - base : nf;
+            {
+                const RegItem it = reg_item(r2 / 2 + 1, cnt);
+                const int f = base + it.f;
+                const long long sm = reg_mode(a, it.m);
+                const SC* src = (f == 0 ? s0 : (f == 1 ? s1 : s2)) + sm;
+                const bool ok = it.on && sm < gd.B;
+                double2* z = reg_line(a, f, it.m);
+                with_radix<L, K>(r1, [&](auto rc) {
+                    constexpr int R = decltype(rc)::value;
+                    SC raw[R];
+#pragma unroll
+                    for (int r = 0; r < R; ++r) {
+                        const int k = it.c + r2 * r, n = k <= P ? k : 2 * P - k;
+                        raw[r] = ok ? src[gd.B * n] : from_c64<SC>(czero());
+                    }
+                    double2 v[R];
+#pragma unroll
+                    for (int r = 0; r < R; ++r) v[r] = to_c64(raw[r]);
+                    reg_column<R>(a, it, z, v);
+                });
+            }
+            reg_sync();
+            {
+                const RegItem it = reg_item(r1 / 2 + 1, cnt);
+                double2* z = reg_line(a, base + it.f, it.m);
+                with_radix<L, K>(r2, [&](auto rc) {
+                    constexpr int R = decltype(rc)::value;
+                    double2 v[R];
+                    reg_row<R>(a, it, z, v);
+                    reg_sync();  // every row is read: the lines are reused
+#pragma unroll
+                    for (int p = 0; p < R; ++p) {
+                        const int n = reg_out(a, it, p);
+                        if (n >= 0) z[n] = v[p];
+                    }
+                });
+            }
+            reg_sync();
+        }
+    }
+    // fields get(i) (coefficients, i < nfields) -> values at the Lobatto points
+    // in dst(i)
+    template <typename SC, typename GetF, typename Dst>
+    __device__ __forceinline__ void dct_inverse_reg(const YArgs& a, const Group<L, K>& g, int nfields, GetF get, Dst dst) {
+        const int P = gd.P, r1 = a.r1, r2 = a.r2, nf = a.nf;
+#pragma unroll 1
+        for (int base = 0; base < nfields; base += nf) {
+            const int cnt = nfields - base < nf ? nfields - base : nf;
+#pragma unroll 1
+            for (int i = 0; i < cnt; ++i) {
+                const CVec<K> x = get(base + i);
+                double2* z = reg_line(a, i, line_slot());
+#pragma unroll
+                for (int e = 0; e < K; ++e) {
+                    const int n = K * g.t + e;
+                    if (n <= P) z[n] = (n == 0 || n == P) ? cscale(x.v[e], 2.0) : x.v[e];
+                }
+            }
+            reg_sync();
+            {
+                const RegItem it = reg_item(r2 / 2 + 1, cnt);
+                double2* z = reg_line(a, it.f, it.m);
+                with_radix<L, K>(r1, [&](auto rc) {
+                    constexpr int R = decltype(rc)::value;
+                    double2 v[R];
+#pragma unroll
+                    for (int r = 0; r < R; ++r) {
+                        const int k = it.c + r2 * r, n = k <= P ? k : 2 * P - k;
+                        v[r] = it.on ? z[n] : czero();
+                    }
+                    reg_sync();  // every column is read: the lines are reused
+                    reg_column<R>(a, it, z, v);
+                });
+            }
+            reg_sync();
+            {
+                const RegItem it = reg_item(r1 / 2 + 1, cnt);
+                double2* z = reg_line(a, it.f, it.m);
+                SC* d0 = dst(base);
+                SC* d1 = dst(base + 1);
+                SC* d2 = dst(base + 2);
+                const long long sm = reg_mode(a, it.m);
+                SC* d = (it.f == 0 ? d0 : (it.f == 1 ? d1 : d2)) + sm;
+                const bool ok = sm < gd.B;
+                with_radix<L, K>(r2, [&](auto rc) {
+                    constexpr int R = decltype(rc)::value;
+                    double2 v[R];
+                    reg_row<R>(a, it, z, v);
+#pragma unroll
+                    for (int p = 0; p < R; ++p) {
+                        const int n = reg_out(a, it, p);
+                        if (ok && n >= 0) d[gd.B * n] = from_c64<SC>(cscale(v[p], 0.5));
+                    }
+                });
+            }
+            reg_sync();
+        }
+    }
 };
 
 // LDS slots of one wave's region: two FFT lines per mode, or the solve's
@@ -200,6 +437,12 @@ struct Tile {
 template <int L, int K>
 __host__ __device__ constexpr int y_region_slots(int ld) {
     return (2 * (64 / L) * ld > 3 * K * 64) ? 2 * (64 / L) * ld : 3 * K * 64;
+}
+
+// the register DCT's region: `fields` lines per mode, or the stash
+template <int L, int K>
+__host__ __device__ constexpr int y_reg_slots(int fields, int zs) {
+    return (fields * (64 / L) * zs > 3 * K * 64) ? fields * (64 / L) * zs : 3 * K * 64;
 }
 
 // Block prologue of every y kernel: the DCT twiddle table and the
@@ -307,6 +550,53 @@ __device__ __forceinline__ void inverse_six(Tile<L, K>& tile, const YArgs& a, co
     }
     tile.template dct_inverse<SC, INPLACE>(out6[3], a.dct, g, W);
     tile.template dct_inverse<SC, INPLACE>(out6[1], a.dct, g, V1);
+}
+
+// inverse_six with the register DCT: the form's fields in passes of a.nf.  The
+// velocity is read back from a.U for every field (a stage has just stored it:
+// L2), not held in registers across the transforms.
+template <int L, int K, typename SC>
+__device__ __forceinline__ void inverse_six_reg(Tile<L, K>& tile, const YArgs& a, const Group<L, K>& g, const ModeInfo& mi) {
+    const int form = a.form;
+    const int nfields = form == FORM_ROTATING ? 5 : (form == FORM_CONVECTIVE ? 6 : 3);
+    // field i of the sequence: rotating V0, Omega_z, V2, Omega_x, V1;
+    // convective V0, dV0, V1, dV1, V2, dV2; divergence V0, V1, V2
+    auto get = [&](int i) {
+        const int c = form == FORM_DIVERGENCE ? i : (form == FORM_CONVECTIVE ? i >> 1 : (i < 2 ? 0 : (i < 4 ? 2 : 1)));
+        CVec<K> x = tile.reload(c == 0 ? a.U[0] : (c == 1 ? a.U[1] : a.U[2]), g);
+        if (c == 0 && mi.mean && mi.valid) {
+#pragma unroll
+            for (int e = 0; e < K; ++e) {
+                const int n = K * g.t + e;
+                if (n < a.gd.Ny) x.v[e] = cadd(x.v[e], cmk(a.base[n], 0.0));
+            }
+        }
+        if (form == FORM_DIVERGENCE || !(i & 1)) return x;
+        x = cheb_deriv(g, x);
+        if (form == FORM_ROTATING) {
+            const CVec<K> v1 = tile.reload(a.U[1], g);
+#pragma unroll
+            for (int e = 0; e < K; ++e) {
+                const double2 d = x.v[e];
+                x.v[e] = i == 1 ? csub(cmuli(cscale(v1.v[e], mi.kx)), d)   // i k V2 - dy V1
+                                : csub(d, cmuli(cscale(v1.v[e], mi.kz)));  // dy V3 - i l V2
+            }
+        }
+        return x;
+    };
+    auto dst = [&](int i) {
+        const int slot = form == FORM_DIVERGENCE ? i
+                         : form == FORM_CONVECTIVE ? (i >> 1) + 3 * (i & 1)
+                                                   : (i == 1 ? 5 : (i == 4 ? 1 : i));
+        double2* d = a.out6[0];
+        if (slot == 1) d = a.out6[1];
+        if (slot == 2) d = a.out6[2];
+        if (slot == 3) d = a.out6[3];
+        if (slot == 4) d = a.out6[4];
+        if (slot == 5) d = a.out6[5];
+        return reinterpret_cast<SC*>(d);
+    };
+    tile.template dct_inverse_reg<SC>(a, g, nfields, get, dst);
 }
 
 // ---------------------------------------------------------------------------
@@ -466,11 +756,13 @@ __device__ __forceinline__ CVec<K> laplacian(const Group<L, K>& g, const CVec<K>
 // Stokes solve, state write, inverse transforms for the next stage.
 // ---------------------------------------------------------------------------
 // SC: storage of the y-physical fields (double2; float2 in the mixed step).
-template <int L, int K, typename SC>
+// REG: the DCTs run in two register radices (a.r1, a.r2), all three nonlinear
+// terms first (their coefficients wait in the LDS lines).
+template <int L, int K, typename SC, bool REG>
 __device__ __forceinline__ void ystage_body(const YArgs& a, unsigned block) {
     extern __shared__ double2 smem[];
     load_tables<L, K>(smem, a);
-    Tile<L, K> tile(a.gd, smem, a.dct.n, a.ld, y_region_slots<L, K>(a.ld), block);
+    Tile<L, K> tile(a.gd, smem, a.dct.n, a.ld, REG ? y_reg_slots<L, K>(3, a.zs) : y_region_slots<L, K>(a.ld), block);
     if (a.order.on) tile.order_modes(a.order);
     Group<L, K> g(tile.tab);
     ModeInfo mi = mode_info(a.gd, tile.s);
@@ -480,6 +772,11 @@ __device__ __forceinline__ void ystage_body(const YArgs& a, unsigned block) {
     // Per component: forward DCT of the nonlinear term, Q = N (stage 1) or
     // A_j Q + N, R_c = lambda U_c + nu Lap U_c - d_c P + (B_j/C_j) Q_c.
     double gold0 = a.c0, gold1 = a.c1;
+    if constexpr (REG) {
+        if (!a.Ncoef[0])  // the three terms come in one form
+            tile.dct_forward_reg(a, reinterpret_cast<const SC*>(a.Nphys[0]), reinterpret_cast<const SC*>(a.Nphys[1]),
+                                 reinterpret_cast<const SC*>(a.Nphys[2]));
+    }
     CVec<K> Pold = tile.load(a.P, g);
     CVec<K> R[3];
 #pragma unroll
@@ -487,6 +784,14 @@ __device__ __forceinline__ void ystage_body(const YArgs& a, unsigned block) {
         CVec<K> Qc;
         if (a.Ncoef[c]) {
             Qc = tile.load(a.Ncoef[c], g);
+        } else if constexpr (REG) {
+            const double2* line = tile.reg_line(a, c, tile.line_slot());
+#pragma unroll
+            for (int e = 0; e < K; ++e) {
+                const int n = K * g.t + e;
+                const double w = ((n == 0 || n == a.gd.P) ? 0.5 * a.norm : a.norm) * a.nl_sign;
+                Qc.v[e] = (n < Ny && !mi.nyq) ? cscale(line[n], w) : czero();
+            }
         } else {
             Qc = tile.dct_forward(reinterpret_cast<const SC*>(a.Nphys[c]), a.dct, a.norm, g, mi.nyq);
 #pragma unroll
@@ -544,6 +849,7 @@ __device__ __forceinline__ void ystage_body(const YArgs& a, unsigned block) {
         }
     }
     double2* st = tile.stash;
+    if constexpr (REG) tile.reg_sync();  // the stash aliases the lines of the nonlinear terms
     stash(st, g, R[0]);
     stash(st + K * L, g, R[1]);
     stash(st + 2 * K * L, g, R[2]);
@@ -562,12 +868,16 @@ __device__ __forceinline__ void ystage_body(const YArgs& a, unsigned block) {
     } else {
         solve_nonzero(g, a, a.bank, mi, st, st + K * L, st + 2 * K * L, Un, Pn);
     }
-    wave_sync();  // the stash aliases the wave's FFT lines reused below
+    if constexpr (REG) tile.reg_sync();  // the stash aliases the FFT lines reused below
+    else wave_sync();
     tile.store(a.U[0], g, Un[0]);
     tile.store(a.U[1], g, Un[1]);
     tile.store(a.U[2], g, Un[2]);
     tile.store(a.P, g, Pn);
-    if (a.out6[0]) inverse_six<L, K, SC>(tile, a, g, mi, [&](int c) { return Un[c]; });
+    if (a.out6[0]) {
+        if constexpr (REG) inverse_six_reg<L, K, SC>(tile, a, g, mi);
+        else inverse_six<L, K, SC>(tile, a, g, mi, [&](int c) { return Un[c]; });
+    }
 }
 
 // Nyquist modes of a stage under the non-Nyquist-first order, elementwise
@@ -605,7 +915,7 @@ __device__ __forceinline__ void ystage_nyquist(const YArgs& a, unsigned blk) {
     }
 }
 
-template <int L, int K, typename SC>
+template <int L, int K, typename SC, bool REG>
 // two waves per SIMD (<= 256 registers per lane): one wave per SIMD leaves
 // the wave-serial scans and LDS FFTs unhidden.  K = 6 and 8 (Ny above 256)
 // keep 1.5 and 2 times the coefficients per lane and run one wave per SIMD,
@@ -619,20 +929,24 @@ __global__ void __launch_bounds__(YNT) __attribute__((amdgpu_waves_per_eu(K >= 6
         }
         // z rows of Nxh modes leave the blocks' row segments unaligned to
         // cache lines: neighbouring blocks share lines, so they run on one XCD
-        ystage_body<L, K, SC>(a, a.order.xcd ? xcd_logical(blockIdx.x, a.order.nyq_first) : blockIdx.x);
+        ystage_body<L, K, SC, REG>(a, a.order.xcd ? xcd_logical(blockIdx.x, a.order.nyq_first) : blockIdx.x);
         return;
     }
-    ystage_body<L, K, SC>(a, blockIdx.x);
+    ystage_body<L, K, SC, REG>(a, blockIdx.x);
 }
 
 // prologue: state U -> six y-physical fields (velocity and vorticity)
-template <int L, int K, typename SC>
+template <int L, int K, typename SC, bool REG>
 __device__ __forceinline__ void yprologue_body(const YArgs& a, unsigned block) {
     extern __shared__ double2 smem[];
     load_tables<L, K>(smem, a);
-    Tile<L, K> tile(a.gd, smem, a.dct.n, a.ld, y_region_slots<L, K>(a.ld), block);
+    Tile<L, K> tile(a.gd, smem, a.dct.n, a.ld, REG ? a.nf * (64 / L) * a.zs : y_region_slots<L, K>(a.ld), block);
     Group<L, K> g(tile.tab);
     ModeInfo mi = mode_info(a.gd, tile.s);
+    if constexpr (REG) {
+        inverse_six_reg<L, K, SC>(tile, a, g, mi);
+        return;
+    }
     inverse_six<L, K, SC>(tile, a, g, mi, [&](int c) { return tile.load(a.U[c], g); });
 }
 
@@ -645,7 +959,8 @@ __device__ __forceinline__ void yprologue_body(const YArgs& a, unsigned block) {
 // INPLACE: the DCT lines are transformed in place (one line per mode, half
 // the LDS of the two-buffer form, so more blocks per CU); the host picks it
 // where the plan fits 8 points per lane (fft_inplace_fits)
-template <int L, int K, typename SC, bool INPLACE = false>
+// REG: the DCTs in two register radices, instead of both
+template <int L, int K, typename SC, bool INPLACE = false, bool REG = false>
 __global__ void __launch_bounds__(YNT) yprologue_kernel(YArgs a) {
     extern __shared__ double2 smem[];
     load_tables<L, K>(smem, a);
@@ -653,11 +968,14 @@ __global__ void __launch_bounds__(YNT) yprologue_kernel(YArgs a) {
     // argument, or a copy of the whole struct, lands in scratch)
     const bool ordered = a.order.on != 0;
     const unsigned block = (ordered && a.order.xcd) ? xcd_logical(blockIdx.x, gridDim.x) : blockIdx.x;
-    Tile<L, K> tile(a.gd, smem, a.dct.n, a.ld, INPLACE ? (64 / L) * a.ld : y_region_slots<L, K>(a.ld), block);
+    Tile<L, K> tile(a.gd, smem, a.dct.n, a.ld,
+                    REG ? a.nf * (64 / L) * a.zs : (INPLACE ? (64 / L) * a.ld : y_region_slots<L, K>(a.ld)), block);
     if (ordered) tile.order_modes(a.order.nreg, a.order.nxr, a.order.zskip);
     Group<L, K> g(tile.tab);
     ModeInfo mi = mode_info(a.gd, tile.s);
-    if constexpr (L == 4) {  // all loads first: the 4-lane build stays within 128 registers so
+    if constexpr (REG) {
+        inverse_six_reg<L, K, SC>(tile, a, g, mi);
+    } else if constexpr (L == 4) {  // all loads first: the 4-lane build stays within 128 registers so
         CVec<K> U[3];
 #pragma unroll
         for (int c = 0; c < 3; ++c) U[c] = tile.load(a.U[c], g);
@@ -670,18 +988,18 @@ __global__ void __launch_bounds__(YNT) yprologue_kernel(YArgs a) {
 // Batched ensemble launches: instance i owns blocks [start[i], start[i+1])
 // of the grid and its own argument block tab[i] (grid, factors, fields).
 // All instances of one launch share the group size L.
-template <int L, int K>
+template <int L, int K, bool REG>
 __global__ void __launch_bounds__(YNT) __attribute__((amdgpu_waves_per_eu(2)))
 ystage_batch_kernel(const YArgs* __restrict__ tab, const unsigned* __restrict__ start, int n) {
     const int i = batch_instance(start, n, blockIdx.x);
-    ystage_body<L, K, double2>(tab[i], blockIdx.x - start[i]);
+    ystage_body<L, K, double2, REG>(tab[i], blockIdx.x - start[i]);
 }
 
-template <int L, int K>
+template <int L, int K, bool REG>
 __global__ void __launch_bounds__(YNT) yprologue_batch_kernel(const YArgs* __restrict__ tab,
                                                               const unsigned* __restrict__ start, int n) {
     const int i = batch_instance(start, n, blockIdx.x);
-    yprologue_body<L, K, double2>(tab[i], blockIdx.x - start[i]);
+    yprologue_body<L, K, double2, REG>(tab[i], blockIdx.x - start[i]);
 }
 
 // Stokes solve! of a bank: R (3 spectral) -> U (3), P (stokes.jl:81-108)
@@ -1136,43 +1454,49 @@ hipError_t launch_y_step(int which, const YArgs& a, hipStream_t st);
 template <int L, int K>
 hipError_t launch_y(int which, const YArgs& a, hipStream_t st);
 template <int L>
-hipError_t launch_y_batch(int which, const YArgs* tab, const unsigned* start, int n, unsigned nblocks, size_t lds,
+hipError_t launch_y_batch(int which, bool reg, const YArgs* tab, const unsigned* start, int n, unsigned nblocks, size_t lds,
                           hipStream_t st);
 
 #if CF_Y_PART != 0
+template <typename Kern>
+static hipError_t y_go(Kern kernel, dim3 grid, size_t lds, const YArgs& a, hipStream_t st) {
+    allow_lds(kernel, lds);
+    hipLaunchKernelGGL(kernel, grid, dim3(YNT), lds, st, a);
+    return hipGetLastError();
+}
 template <int L, int K>
 hipError_t launch_y_step(int which, const YArgs& a, hipStream_t st) {
     constexpr int M = YNT / L;
-    const dim3 grid((unsigned)((a.gd.B + M - 1) / M));
+    if (which != Y_STAGE && which != Y_PROLOGUE) return hipErrorInvalidValue;
     const size_t lds = y_lds_lk<L, K>(a.gd.Ny, a.ld);
+    const size_t tables = (2 * (size_t)(a.gd.Ny - 1) + (size_t)CHEB_TAB_ARRAYS * K * L / 2) * sizeof(double2);
     YArgs b = a;
-    if (which == Y_STAGE) {
-        allow_lds(ystage_kernel<L, K, double2>, lds);
-        allow_lds(ystage_kernel<L, K, float2>, lds);
-        const unsigned nb = y_stage_order<L>(b);
-        const dim3 g2 = nb ? dim3(nb) : grid;
-        if (a.mixed) hipLaunchKernelGGL((ystage_kernel<L, K, float2>), g2, dim3(YNT), lds, st, b);
-        else hipLaunchKernelGGL((ystage_kernel<L, K, double2>), g2, dim3(YNT), lds, st, b);
-    } else if (which == Y_PROLOGUE) {
-        // regular (non-Nyquist) blocks only, see yprologue_kernel
-        const dim3 g2 = y_stage_order<L>(b) ? dim3(b.order.nyq_first) : grid;
-        if (fft_inplace_fits(a.dct, 64 / L, 8, 64)) {
-            const size_t ldsi = (2 * (size_t)(a.gd.Ny - 1) + (size_t)CHEB_TAB_ARRAYS * K * L / 2 +
-                                 (YNT / 64) * (size_t)(64 / L) * a.ld) * sizeof(double2);
-            allow_lds(yprologue_kernel<L, K, double2, true>, ldsi);
-            allow_lds(yprologue_kernel<L, K, float2, true>, ldsi);
-            if (a.mixed) hipLaunchKernelGGL((yprologue_kernel<L, K, float2, true>), g2, dim3(YNT), ldsi, st, b);
-            else hipLaunchKernelGGL((yprologue_kernel<L, K, double2, true>), g2, dim3(YNT), ldsi, st, b);
-            return hipGetLastError();
+    const unsigned nb = y_stage_order<L>(b);
+    // the prologue runs the regular (non-Nyquist) blocks only, see yprologue_kernel
+    const dim3 grid(!nb ? (unsigned)((a.gd.B + M - 1) / M) : (which == Y_STAGE ? nb : b.order.nyq_first));
+    if constexpr (y_has_reg<L, K>()) {
+        y_reg_split(b, L, K);
+        if (b.r1) {
+            if (which == Y_STAGE)
+                return y_go(ystage_kernel<L, K, double2, true>, grid, y_reg_lds(b, L, K), b, st);
+            // K = 6: the register prologue runs one wave per SIMD (54 AGPRs), the
+            // staged one three (256x257x256: 1087 against 823 us)
+            if constexpr (K == 4) {
+                const size_t ldsr = tables + (YNT / 64) * (size_t)b.nf * (64 / L) * b.zs * sizeof(double2);
+                return y_go(yprologue_kernel<L, K, double2, false, true>, grid, ldsr, b, st);
+            }
         }
-        allow_lds(yprologue_kernel<L, K, double2>, lds);
-        allow_lds(yprologue_kernel<L, K, float2>, lds);
-        if (a.mixed) hipLaunchKernelGGL((yprologue_kernel<L, K, float2>), g2, dim3(YNT), lds, st, b);
-        else hipLaunchKernelGGL((yprologue_kernel<L, K, double2>), g2, dim3(YNT), lds, st, b);
-    } else {
-        return hipErrorInvalidValue;
     }
-    return hipGetLastError();
+    if (which == Y_STAGE)
+        return a.mixed ? y_go(ystage_kernel<L, K, float2, false>, grid, lds, b, st)
+                       : y_go(ystage_kernel<L, K, double2, false>, grid, lds, b, st);
+    if (fft_inplace_fits(a.dct, 64 / L, 8, 64)) {
+        const size_t ldsi = tables + (YNT / 64) * (size_t)(64 / L) * a.ld * sizeof(double2);
+        return a.mixed ? y_go(yprologue_kernel<L, K, float2, true>, grid, ldsi, b, st)
+                       : y_go(yprologue_kernel<L, K, double2, true>, grid, ldsi, b, st);
+    }
+    return a.mixed ? y_go(yprologue_kernel<L, K, float2>, grid, lds, b, st)
+                   : y_go(yprologue_kernel<L, K, double2>, grid, lds, b, st);
 }
 
 template <int L, int K>
@@ -1203,19 +1527,23 @@ hipError_t launch_y(int which, const YArgs& a, hipStream_t st) {
     return hipGetLastError();
 }
 
-template <int L>
-hipError_t launch_y_batch(int which, const YArgs* tab, const unsigned* start, int n, unsigned nblocks, size_t lds,
-                                 hipStream_t st) {
-    if (which == Y_STAGE) {
-        allow_lds(ystage_batch_kernel<L, 4>, lds);
-        hipLaunchKernelGGL((ystage_batch_kernel<L, 4>), dim3(nblocks), dim3(YNT), lds, st, tab, start, n);
-    } else if (which == Y_PROLOGUE) {
-        allow_lds(yprologue_batch_kernel<L, 4>, lds);
-        hipLaunchKernelGGL((yprologue_batch_kernel<L, 4>), dim3(nblocks), dim3(YNT), lds, st, tab, start, n);
-    } else {
-        return hipErrorInvalidValue;
-    }
+template <typename Kern>
+static hipError_t y_go_batch(Kern kernel, const YArgs* tab, const unsigned* start, int n, unsigned nblocks, size_t lds,
+                             hipStream_t st) {
+    allow_lds(kernel, lds);
+    hipLaunchKernelGGL(kernel, dim3(nblocks), dim3(YNT), lds, st, tab, start, n);
     return hipGetLastError();
+}
+template <int L>
+hipError_t launch_y_batch(int which, bool reg, const YArgs* tab, const unsigned* start, int n, unsigned nblocks, size_t lds,
+                          hipStream_t st) {
+    if (which == Y_STAGE)
+        return reg ? y_go_batch(ystage_batch_kernel<L, 4, true>, tab, start, n, nblocks, lds, st)
+                   : y_go_batch(ystage_batch_kernel<L, 4, false>, tab, start, n, nblocks, lds, st);
+    if (which == Y_PROLOGUE)
+        return reg ? y_go_batch(yprologue_batch_kernel<L, 4, true>, tab, start, n, nblocks, lds, st)
+                   : y_go_batch(yprologue_batch_kernel<L, 4, false>, tab, start, n, nblocks, lds, st);
+    return hipErrorInvalidValue;
 }
 
 #endif  // CF_Y_PART != 0
@@ -1276,14 +1604,41 @@ size_t y_lds_bytes_layout(int Ny, int ld, int L, int K) {
     return 0;
 }
 
-hipError_t launch_ykernel_batch(int which, int L, const YArgs* tab, const unsigned* start, int n, unsigned nblocks,
+// The split whose larger radix is smallest (registers), the smaller one first;
+// the columns and rows of one field must fit the lanes.  The mixed step keeps
+// the staged transforms and their bits: a last-bit difference before the FP32
+// rounding of a field flips some of its values by an FP32 ulp, and the register
+// form gains nothing there (256x193x256: 7.84 ms staged, 7.95).
+void y_reg_split(YArgs& a, int L, int K) {
+    const int N = 2 * a.gd.P, W = 64 / L;
+    const bool staged = a.r1 < 0;
+    a.r1 = a.r2 = a.nf = a.zs = 0;
+    if (a.mixed || staged) return;
+    for (int r2 = 2; r2 <= 32; ++r2) {
+        if (N % r2 != 0 || N / r2 > r2 || !y_radix(L, K, r2) || !y_radix(L, K, N / r2)) continue;
+        const int nf = 64 / (W * (r2 / 2 + 1)), lines = (N / r2 / 2 + 1) * (r2 | 1);
+        if (nf < 1) return;
+        a.r1 = N / r2;
+        a.r2 = r2;
+        a.nf = nf < 3 ? nf : 3;
+        a.zs = (lines > a.gd.Ny ? lines : a.gd.Ny) | 1;
+        return;
+    }
+}
+size_t y_reg_lds(const YArgs& a, int L, int K) {
+    const int W = 64 / L, lines = 3 * W * a.zs, stash = 3 * K * 64;
+    return (2 * (size_t)a.gd.P + (size_t)CHEB_TAB_ARRAYS * K * L / 2 + (YNT / 64) * (size_t)(lines > stash ? lines : stash)) *
+           sizeof(double2);
+}
+
+hipError_t launch_ykernel_batch(int which, int L, bool reg, const YArgs* tab, const unsigned* start, int n, unsigned nblocks,
                                 size_t lds, hipStream_t st) {
     switch (L) {
-        case 4: return launch_y_batch<4>(which, tab, start, n, nblocks, lds, st);
-        case 8: return launch_y_batch<8>(which, tab, start, n, nblocks, lds, st);
-        case 16: return launch_y_batch<16>(which, tab, start, n, nblocks, lds, st);
-        case 32: return launch_y_batch<32>(which, tab, start, n, nblocks, lds, st);
-        case 64: return launch_y_batch<64>(which, tab, start, n, nblocks, lds, st);
+        case 4: return launch_y_batch<4>(which, reg, tab, start, n, nblocks, lds, st);
+        case 8: return launch_y_batch<8>(which, reg, tab, start, n, nblocks, lds, st);
+        case 16: return launch_y_batch<16>(which, reg, tab, start, n, nblocks, lds, st);
+        case 32: return launch_y_batch<32>(which, reg, tab, start, n, nblocks, lds, st);
+        case 64: return launch_y_batch<64>(which, reg, tab, start, n, nblocks, lds, st);
         default: return hipErrorInvalidValue;
     }
 }
@@ -1321,18 +1676,18 @@ hipError_t launch_ykernel(int which, const YArgs& a, hipStream_t st) {
 #if CF_Y_PART == 1
 template hipError_t launch_y<4, 4>(int, const YArgs&, hipStream_t);
 template hipError_t launch_y<8, 4>(int, const YArgs&, hipStream_t);
-template hipError_t launch_y_batch<4>(int, const YArgs*, const unsigned*, int, unsigned, size_t, hipStream_t);
-template hipError_t launch_y_batch<8>(int, const YArgs*, const unsigned*, int, unsigned, size_t, hipStream_t);
+template hipError_t launch_y_batch<4>(int, bool, const YArgs*, const unsigned*, int, unsigned, size_t, hipStream_t);
+template hipError_t launch_y_batch<8>(int, bool, const YArgs*, const unsigned*, int, unsigned, size_t, hipStream_t);
 #elif CF_Y_PART == 2
 template hipError_t launch_y<16, 4>(int, const YArgs&, hipStream_t);
 template hipError_t launch_y_step<16, 8>(int, const YArgs&, hipStream_t);
-template hipError_t launch_y_batch<16>(int, const YArgs*, const unsigned*, int, unsigned, size_t, hipStream_t);
+template hipError_t launch_y_batch<16>(int, bool, const YArgs*, const unsigned*, int, unsigned, size_t, hipStream_t);
 #elif CF_Y_PART == 3
 template hipError_t launch_y<32, 4>(int, const YArgs&, hipStream_t);
-template hipError_t launch_y_batch<32>(int, const YArgs*, const unsigned*, int, unsigned, size_t, hipStream_t);
+template hipError_t launch_y_batch<32>(int, bool, const YArgs*, const unsigned*, int, unsigned, size_t, hipStream_t);
 #elif CF_Y_PART == 4
 template hipError_t launch_y<64, 4>(int, const YArgs&, hipStream_t);
-template hipError_t launch_y_batch<64>(int, const YArgs*, const unsigned*, int, unsigned, size_t, hipStream_t);
+template hipError_t launch_y_batch<64>(int, bool, const YArgs*, const unsigned*, int, unsigned, size_t, hipStream_t);
 #elif CF_Y_PART == 5
 template hipError_t launch_y_step<32, 8>(int, const YArgs&, hipStream_t);
 #elif CF_Y_PART == 6

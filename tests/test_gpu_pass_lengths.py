@@ -59,3 +59,24 @@ def test_x_lengths_step(gpu, Nx, form):
     say("x length step", form, Nx)
     U, P, Ur, Pr, _, _, env = run_pair(gpu, (Nx, 9, 6), 1, form=form)
     assert_parity(f"step {form} {Nx}", _split((U, P)), _split((Ur, Pr)), env)
+
+
+# each pair of register radices of the wall-normal transform (2 x 4 .. 24 x 24, 16 x 32), one to three fields a
+# pass, the edges of the lane layouts, and a length that keeps the staged transform (197)
+NY = [5, 7, 9, 13, 17, 19, 21, 25, 29, 31, 33, 37, 43, 49, 51, 57, 61, 65, 73, 81, 85, 91, 97, 101, 109, 113, 121, 127,
+      129, 141, 145, 151, 161, 163, 181, 193, 197, 211, 241, 253, 257, 289, 321, 337]
+
+
+@pytest.mark.parametrize("Ny", NY)
+def test_y_lengths_step(gpu, Ny):
+    say("y length step", Ny)
+    U, P, Ur, Pr, _, _, env = run_pair(gpu, (8, Ny, 7), 1)
+    assert_parity(f"step {Ny}", _split((U, P)), _split((Ur, Pr)), env)
+
+
+@pytest.mark.parametrize("form", ["convective", "divergence"])
+@pytest.mark.parametrize("Ny", [9, 17, 33, 49, 65, 97, 101, 129, 193, 257])
+def test_y_lengths_forms(gpu, Ny, form):
+    say("y length form", form, Ny)
+    U, P, Ur, Pr, _, _, env = run_pair(gpu, (7, Ny, 8), 1, form=form)
+    assert_parity(f"step {form} {Ny}", _split((U, P)), _split((Ur, Pr)), env)
