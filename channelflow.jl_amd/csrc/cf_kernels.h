@@ -184,7 +184,7 @@ size_t y_reg_lds(const YArgs& a, int L, int K);  // LDS bytes of that launch
 hipError_t launch_zpass(int dir, const ZArgs& a, hipStream_t st);
 size_t z_lds_bytes(const ZArgs& a);
 int z_inplace_ppt(const FFTPlan& plan, int KT);  // 0: the plan needs two buffers
-bool reg_radix(int r);                           // radices built in registers
+bool reg_radix(int r);                           // radices of the register z pass
 bool z_reg_split(int n, int* r1, int* r2);       // false: n = r1 r2 has no such split
 hipError_t launch_zreg(int dir, const ZArgs& a, hipStream_t st);
 int z_reg_class(const ZArgs& a);    // register class of the kernel: radices up to 12, 16 or 24

@@ -13,10 +13,32 @@ namespace cf {
 
 // cos and sin of 2 pi t / R, correctly rounded
 template <int R> struct RegTwiddle;
+template <> struct RegTwiddle<3> {
+    static constexpr double c[3] = {1.0, -0.5, -0.5};
+    static constexpr double s[3] = {0.0, 0.8660254037844386, -0.8660254037844386};
+};
+template <> struct RegTwiddle<5> {
+    static constexpr double c[5] = {1.0, 0.30901699437494745, -0.8090169943749475, -0.8090169943749475,
+        0.30901699437494745};
+    static constexpr double s[5] = {0.0, 0.9510565162951535, 0.5877852522924731, -0.5877852522924731,
+        -0.9510565162951535};
+};
 template <> struct RegTwiddle<6> {
     static constexpr double c[6] = {1.0, 0.5, -0.5, -1.0, -0.5, 0.5};
     static constexpr double s[6] = {0.0, 0.8660254037844386, 0.8660254037844386, 0.0, -0.8660254037844386,
         -0.8660254037844386};
+};
+template <> struct RegTwiddle<7> {
+    static constexpr double c[7] = {1.0, 0.6234898018587335, -0.2225209339563144, -0.9009688679024191,
+        -0.9009688679024191, -0.2225209339563144, 0.6234898018587335};
+    static constexpr double s[7] = {0.0, 0.7818314824680298, 0.9749279121818236, 0.4338837391175581,
+        -0.4338837391175581, -0.9749279121818236, -0.7818314824680298};
+};
+template <> struct RegTwiddle<8> {
+    static constexpr double c[8] = {1.0, 0.7071067811865476, 0.0, -0.7071067811865476, -1.0,
+        -0.7071067811865476, 0.0, 0.7071067811865476};
+    static constexpr double s[8] = {0.0, 0.7071067811865476, 1.0, 0.7071067811865476, 0.0, -0.7071067811865476,
+        -1.0, -0.7071067811865476};
 };
 template <> struct RegTwiddle<9> {
     static constexpr double c[9] = {1.0, 0.766044443118978, 0.17364817766693036, -0.5, -0.9396926207859084,
@@ -276,6 +298,128 @@ __device__ __forceinline__ void dft_reg(double2* v, int dir) {
 #pragma unroll
             for (int s = 0; s < B; ++s) v[p + A * s] = t[s];
         }
+    }
+}
+
+// half-length packing of an even R, M = R/2: Z_k = E + i O with E = g_k + conj
+// g_{M-k}, O = (g_k - conj g_{M-k}) exp(2 pi i k / R); Z_{M-k} = conj E + i conj O
+template <int R, int K>
+__device__ __forceinline__ void c2r_pack(const double2* g, double2* z) {
+#pragma clang fp contract(off)
+    constexpr int M = R / 2;
+    if constexpr (2 * K < M) {
+        const double2 a = g[K], b = cconj(g[M - K]);
+        const double2 e = cadd(a, b), o = reg_twiddle<R, K>(csub(a, b), +1);
+        z[K] = cmk(e.x - o.y, e.y + o.x);
+        z[M - K] = cmk(e.x + o.y, o.x - e.y);
+        c2r_pack<R, K + 1>(g, z);
+    } else if constexpr (2 * K == M) {
+        z[K] = cmk(2.0 * g[K].x, -2.0 * g[K].y);
+    }
+}
+// its inverse: g_k = (E - i O) / 2 with E = Z_k + conj Z_{M-k}, O = (Z_k - conj
+// Z_{M-k}) exp(-2 pi i k / R); g_{M-k} = conj (E + i O) / 2
+template <int R, int K>
+__device__ __forceinline__ void r2c_unpack(const double2* z, double2* g) {
+#pragma clang fp contract(off)
+    constexpr int M = R / 2;
+    if constexpr (2 * K < M) {
+        const double2 a = z[K], b = cconj(z[M - K]);
+        const double2 e = cscale(cadd(a, b), 0.5), o = reg_twiddle<R, K>(cscale(csub(a, b), 0.5), -1);
+        g[K] = cmk(e.x + o.y, e.y - o.x);
+        g[M - K] = cmk(e.x - o.y, -(e.y + o.x));
+        r2c_unpack<R, K + 1>(z, g);
+    } else if constexpr (2 * K == M) {
+        g[K] = cconj(z[K]);
+    }
+}
+
+// Real DFTs: x real of length R, g its R/2 + 1 lowest coefficients (the others
+// are their conjugates).  Every output is a sum over this one line alone, so
+// its error is relative to the line's own size and a zero line stays zero.
+// Odd R: cosine and sine sums; even R: the complex transform of half the
+// length, even points in the real part and odd points in the imaginary part.
+
+// x_s = sum_k g_k exp(2 pi i k s / R); Im g_0, and Im g_{R/2} of an even R, are ignored
+template <int R>
+__device__ __forceinline__ void c2r_reg(const double2* g, double* x) {
+#pragma clang fp contract(off)
+    if constexpr (R == 2) {
+        x[0] = g[0].x + g[1].x;
+        x[1] = g[0].x - g[1].x;
+    } else if constexpr (R % 2 == 1) {
+        constexpr int H = R / 2;
+        double a[H], b[H];
+#pragma unroll
+        for (int k = 0; k < H; ++k) {
+            a[k] = 2.0 * g[1 + k].x;
+            b[k] = 2.0 * g[1 + k].y;
+        }
+        double t = a[0];
+#pragma unroll
+        for (int k = 1; k < H; ++k) t += a[k];
+        x[0] = g[0].x + t;
+#pragma unroll
+        for (int s = 1; s <= H; ++s) {
+            double m = g[0].x, n = b[0] * RegTwiddle<R>::s[s];
+#pragma unroll
+            for (int k = 1; k <= H; ++k) m = fma(a[k - 1], RegTwiddle<R>::c[(k * s) % R], m);
+#pragma unroll
+            for (int k = 2; k <= H; ++k) n = fma(b[k - 1], RegTwiddle<R>::s[(k * s) % R], n);
+            x[s] = m - n;
+            x[R - s] = m + n;
+        }
+    } else {
+        constexpr int M = R / 2;
+        double2 z[M];
+        z[0] = cmk(g[0].x + g[M].x, g[0].x - g[M].x);
+        c2r_pack<R, 1>(g, z);
+        dft_reg<M>(z, +1);
+#pragma unroll
+        for (int m = 0; m < M; ++m) {
+            x[2 * m] = z[m].x;
+            x[2 * m + 1] = z[m].y;
+        }
+    }
+}
+
+// g_k = sum_s x_s exp(-2 pi i k s / R), k <= R/2
+template <int R>
+__device__ __forceinline__ void r2c_reg(const double* x, double2* g) {
+#pragma clang fp contract(off)
+    if constexpr (R == 2) {
+        g[0] = cmk(x[0] + x[1], 0.0);
+        g[1] = cmk(x[0] - x[1], 0.0);
+    } else if constexpr (R % 2 == 1) {
+        constexpr int H = R / 2;
+        double e[H], d[H];
+#pragma unroll
+        for (int s = 0; s < H; ++s) {
+            e[s] = x[1 + s] + x[R - 1 - s];
+            d[s] = x[R - 1 - s] - x[1 + s];
+        }
+        double t = e[0];
+#pragma unroll
+        for (int s = 1; s < H; ++s) t += e[s];
+        g[0] = cmk(x[0] + t, 0.0);
+#pragma unroll
+        for (int k = 1; k <= H; ++k) {
+            double m = x[0], n = d[0] * RegTwiddle<R>::s[k];
+#pragma unroll
+            for (int s = 1; s <= H; ++s) m = fma(e[s - 1], RegTwiddle<R>::c[(k * s) % R], m);
+#pragma unroll
+            for (int s = 2; s <= H; ++s) n = fma(d[s - 1], RegTwiddle<R>::s[(k * s) % R], n);
+            g[k] = cmk(m, n);
+        }
+    } else {
+        constexpr int M = R / 2;
+        double2 z[M];
+#pragma unroll
+        for (int m = 0; m < M; ++m) z[m] = cmk(x[2 * m], x[2 * m + 1]);
+        dft_reg<M>(z, -1);
+        g[0] = cmk(z[0].x + z[0].y, 0.0);
+        g[M] = cmk(z[0].x - z[0].y, 0.0);
+        r2c_unpack<R, 1>(z, g);
     }
 }
 
