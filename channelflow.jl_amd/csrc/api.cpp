@@ -642,10 +642,11 @@ struct NonlinearArgs {
     XArgs x;
 };
 
-// staged: the passes of the setup calls (cf_nonlinear, cf_pressure) keep the
-// staged multi-pass transforms.  An FP32-mixed run amplifies a last-bit change
-// of its initial pressure to FP32 noise within one step, so the calls that
-// prepare it keep their bits; they run once per trajectory.
+// staged: the calls that prepare a mixed run (cf_nonlinear and cf_pressure of a
+// mixed problem) keep the staged multi-pass transforms.  The run amplifies a
+// last-bit change of its initial pressure to FP32 noise within one step, so
+// they keep their bits; they run once per trajectory.  An FP64 problem's calls
+// run the step's own passes.
 static NonlinearArgs nonlinear_args(cf_problem* h, bool mixed, bool staged = false) {
     const GridDims& gd = h->gd;
     double2* six[6];
@@ -1400,8 +1401,9 @@ extern "C" int cf_inverse3(cf_problem* h, const double* U0, const double* U1, co
 
 // nonlinear term of U into spectral N (3 fields)
 static int enqueue_nonlinear_spec(cf_problem* h, double2* const U[3], double2* const N[3], hipStream_t st) {
-    if (int rc = enqueue_prologue(h, U, st, false, true)) return rc;
-    if (int rc = enqueue_nonlinear_phys(h, st, nullptr, false, true)) return rc;
+    const bool staged = h->mixed != 0;
+    if (int rc = enqueue_prologue(h, U, st, false, staged)) return rc;
+    if (int rc = enqueue_nonlinear_phys(h, st, nullptr, false, staged)) return rc;
     if (h->form == CF_FORM_DIVERGENCE) return enqueue_nonlinear_coef(h, N, st);
     YArgs a = base_yargs(h);
     a.nl_sign = (h->form == CF_FORM_CONVECTIVE) ? -1.0 : 1.0;
