@@ -1264,7 +1264,8 @@ __global__ void __launch_bounds__(YNT) ydot_kernel(YArgs a, int curl) {
 #pragma unroll
     for (int c = 0; c < 3; ++c)
 #pragma unroll
-        for (int e = 0; e < K; ++e) acc += u[c].v[e].x * s[c][e].x + u[c].v[e].y * s[c][e].y;  // Re(conj(u_m) (M v)_m)
+        for (int e = 0; e < K; ++e)  // Re(conj(u_m) (M v)_m); s of the padded degrees may be infinite where u is 0
+            if (K * g.t + e < Ny) acc += u[c].v[e].x * s[c][e].x + u[c].v[e].y * s[c][e].y;
     acc = g.sum(acc);
     const bool use = mi.valid && !mi.nyq;
     double* part = reinterpret_cast<double*>(smem);  // twiddle area is free now
