@@ -642,11 +642,10 @@ struct NonlinearArgs {
     XArgs x;
 };
 
-// staged: the calls that prepare a mixed run (cf_nonlinear and cf_pressure of a
-// mixed problem) keep the staged multi-pass transforms.  The run amplifies a
-// last-bit change of its initial pressure to FP32 noise within one step, so
-// they keep their bits; they run once per trajectory.  An FP64 problem's calls
-// run the step's own passes.
+// staged: cf_pressure keeps the staged multi-pass transforms.  An FP32-mixed run
+// amplifies a last-bit change of its initial pressure to FP32 noise within one
+// step, so the pressure keeps its bits, and both precisions give the same ones.
+// It runs once per trajectory.
 static NonlinearArgs nonlinear_args(cf_problem* h, bool mixed, bool staged = false) {
     const GridDims& gd = h->gd;
     double2* six[6];
@@ -1400,8 +1399,8 @@ extern "C" int cf_inverse3(cf_problem* h, const double* U0, const double* U1, co
 }
 
 // nonlinear term of U into spectral N (3 fields)
-static int enqueue_nonlinear_spec(cf_problem* h, double2* const U[3], double2* const N[3], hipStream_t st) {
-    const bool staged = h->mixed != 0;
+static int enqueue_nonlinear_spec(cf_problem* h, double2* const U[3], double2* const N[3], hipStream_t st,
+                                  bool staged = false) {
     if (int rc = enqueue_prologue(h, U, st, false, staged)) return rc;
     if (int rc = enqueue_nonlinear_phys(h, st, nullptr, false, staged)) return rc;
     if (h->form == CF_FORM_DIVERGENCE) return enqueue_nonlinear_coef(h, N, st);
@@ -1512,7 +1511,7 @@ extern "C" int cf_pressure(cf_problem* h, const double* U0, const double* U1, co
     double2* U[3] = {(double2*)U0, (double2*)U1, (double2*)U2};
     double2* A[3];
     for (int i = 0; i < 3; ++i) A[i] = fld(h->R, h->gd.S, i);
-    if (int rc = enqueue_nonlinear_spec(h, U, A, st)) return rc;
+    if (int rc = enqueue_nonlinear_spec(h, U, A, st, true)) return rc;
     YArgs a = base_yargs(h);
     for (int i = 0; i < 3; ++i) a.Rin[i] = A[i];
     a.U[1] = U[1];
