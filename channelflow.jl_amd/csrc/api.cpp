@@ -1665,12 +1665,10 @@ extern "C" int cf_random_state(cf_problem* h, double epsilon, unsigned long long
     return cf_pressure(h, U0, U1, U2, P, stream);
 }
 
-// Tile autotuner of one problem, on its workspaces: times the FP64 z passes of
-// the nonlinear term for each tile width and, where the x pass is staged, its
-// variants and wavefront counts (a mixed problem's FP64 passes are those of
-// its setup calls), the wall-normal layouts, and a mixed step's FP32 x pass,
-// and keeps the fastest.  The results of the x and z passes do not depend on
-// the tiling; the wall-normal layouts agree to roundoff.
+// Tile autotuner of one problem (FP64 step): times the z passes of the
+// nonlinear term for each in-place tile width and the x pass for each
+// wavefront count on the problem's workspaces, and keeps the fastest.  The
+// results of every pass do not depend on the tiling.
 extern "C" int cf_problem_tune(cf_problem* h, void* stream) {
     if (!h) return fail(CF_ERR_ARGUMENT, "null problem");
     DeviceGuard dg(h->device);
@@ -1694,18 +1692,17 @@ extern "C" int cf_problem_tune(cf_problem* h, void* stream) {
         return 0;
     };
     int rc = 0;
-    const bool staged = h->mixed != 0;  // of the FP64 passes (nonlinear_args)
     // z passes: both directions of the form's nonlinear term
     const int keepKT = h->KT, keepPPT = h->zppt;
     int bestKT = keepKT, bestPPT = keepPPT;
     float best = 1e30f;
     for (int kt = 1; kt <= std::min(32, h->gd.Nxh) && !rc; ++kt) {
         const int ppt = z_inplace_ppt(h->pz, kt);
-        if ((!h->zr1 || staged) && !ppt && !(kt == keepKT && keepPPT == 0)) continue;
+        if (!h->zr1 && !ppt && !(kt == keepKT && keepPPT == 0)) continue;
         if (!z_width_ok(h, kt)) continue;
         h->KT = kt;
         h->zppt = ppt;
-        const NonlinearArgs na = nonlinear_args(h, false, staged);
+        const NonlinearArgs na = nonlinear_args(h, false);
         float ms;
         rc = timed([&] {
             HIPTRY(launch_zpass(+1, na.zin, st));
@@ -1720,9 +1717,9 @@ extern "C" int cf_problem_tune(cf_problem* h, void* stream) {
     }
     h->KT = bestKT;
     h->zppt = bestPPT;
-    // staged x pass: wavefronts per block (even padded Nx), and for the
-    // rotating form the six-line, split (three-line) or async variant
-    if (!rc && h->gd.Nxp % 2 == 0 && (!h->xr1 || staged)) {
+    // x pass: wavefronts per block (even padded Nx), and for the rotating
+    // form the six-line or the split (three-line) variant
+    if (!rc && h->gd.Nxp % 2 == 0 && !h->xr1) {
         const int keepSplit = h->xsplit;
         int bestW[3] = {h->xwaves, h->xwavess, h->xwavesa}, bestSplit = keepSplit;
         int* waves[3] = {&h->xwaves, &h->xwavess, &h->xwavesa};
@@ -1733,7 +1730,7 @@ extern "C" int cf_problem_tune(cf_problem* h, void* stream) {
             h->xsplit = split;
             for (int w = 1; w <= maxv[split] && !rc; ++w) {
                 *waves[split] = w;
-                const NonlinearArgs na = nonlinear_args(h, false, staged);
+                const NonlinearArgs na = nonlinear_args(h, false);
                 float ms;
                 rc = timed([&] {
                     HIPTRY(launch_xpass(na.x, st));
