@@ -93,6 +93,7 @@ struct cf_problem {
     int KT = 1, zld = 0, LPB = 1, xld = 0, yld = 0;
     int xwaves = 4;  // even Nxp: wavefronts per block of the nonlinear x pass
     int zppt = 0;    // z pass in-place points per thread (0: two buffers)
+    int KTs = 1, zppts = 0;  // the same of the staged z passes beside register ones
     int zr1 = 0, zr2 = 0;  // register radices of the FP64 z pass (0: none, the staged passes)
     int xr1 = 0, xr2 = 0;  // the same of the FP64 x pass
     int xppt = 0;    // even-Nxp x pass in-place points per lane (0: two buffers)
@@ -427,6 +428,8 @@ extern "C" int cf_problem_create(const cf_config* cfg, cf_problem** out) {
         h->KT = (int)std::max<size_t>(1, std::min<size_t>(16, LDS_MAX / (2 * (size_t)h->zld * sizeof(double2))));
         h->KT = std::min(h->KT, gd.Nxh);
     }
+    h->KTs = h->KT;
+    h->zppts = h->zppt;
     if (h->zr1) {
         // register passes: 256-byte column segments; narrower tiles where the
         // launch would leave CUs without a block, or three blocks would not
@@ -466,8 +469,13 @@ extern "C" int cf_problem_create(const cf_config* cfg, cf_problem** out) {
             h->xppts = x_inplace_ppt(xs);
             xs.ppt = h->xppts;
             h->xwavess = h->xppts ? x_max_waves(xs) : 0;
-            h->xsplit = h->xwavess > 0 ? 1 : 0;
             h->xwavesa = h->xppt ? h->xwaves : 0;  // same LDS lines as the six-line in-place pass
+            // the default: async and all its waves, the fastest or within 3 % of
+            // it from 16x33x16 to 256x193x256 (there pressure takes 2857 us, 3050
+            // with the split variant, 3249 with the six-line one); it serves
+            // cf_pressure untuned, since the tuner leaves the staged variants out
+            // where the step's x pass is in registers
+            h->xsplit = h->xwavesa > 0 ? 2 : (h->xwavess > 0 ? 1 : 0);
         }
         h->xmaxw[0] = h->xwaves;
         h->xmaxw[1] = h->xwavess;
@@ -687,10 +695,17 @@ static NonlinearArgs nonlinear_args(cf_problem* h, bool mixed, bool staged = fal
     }
     const int nout = h->form == CF_FORM_DIVERGENCE ? 6 : 3;
     na.zout = make_zargs(h, nout, zb, six, 0, mixed);
-    if (staged)
-        for (ZArgs* z : {&na.zin, &na.zout}) z->r1 = z->r2 = 0;
-    else if (!mixed)
-        x_registers(h, x);
+    if (staged) {
+        for (ZArgs* z : {&na.zin, &na.zout}) {
+            if (z->r1) {  // the tile width is the register pass's
+                z->KT = h->KTs;
+                z->ppt = h->zppts;
+                z->mul_kt = recip_mul((unsigned)z->KT);
+            }
+            z->r1 = z->r2 = 0;
+        }
+    }
+    if (!staged && !mixed) x_registers(h, x);
     return na;
 }
 
