@@ -27,7 +27,7 @@ __all__ = ["Grid", "ChannelFlowProblem", "CouetteFlow", "PoiseuilleFlow", "State
            "step_", "project_", "pressure", "FFT", "IFFT", "velocity", "stagepressure", "kinetic_energy",
            "require_device", "RotatingForm", "ConvectiveForm", "DivergenceForm", "dot", "norm", "dissipation_rate",
            "power_input", "plane_statistics", "ProfileStatistics", "flow", "device_gaussian_noise",
-           "savefield", "loadfield", "Ensemble", "velocity_gradient", "box_filter", "tune", "get_tiles", "set_tiles"]
+           "savefield", "loadfield", "Ensemble", "velocity_gradient", "box_filter", "tune", "get_tiles", "set_tiles", "transforms"]
 
 # nonlinear forms (src/nonlinear.jl:214-224)
 RotatingForm = "rotating"
@@ -440,9 +440,11 @@ def flow(problem):
 
 
 def tune(problem, stream=None):
-    """Pick the problem's z tile width and x wavefronts per block by timing
-    them on the device (cf_problem_tune); returns (KT, z points per thread,
-    x wavefronts).  Results of the step are identical for any tiling."""
+    """Pick the problem's z tile width, the variant and wavefronts per block of
+    a staged x pass, and the wall-normal layout by timing them on the device
+    (cf_problem_tune); returns (KT, z points per thread, x wavefronts).
+    Results are identical for any x and z tiling; the wall-normal layouts agree
+    to roundoff (set_tiles keeps one for the same bits in every run)."""
     _lib.check(_lib.load().cf_problem_tune(problem.scheme.h, _stream(stream)))
     out = (C.c_int * 3)()
     _lib.check(_lib.load().cf_problem_tiles(problem.scheme.h, out))
@@ -468,12 +470,21 @@ def set_tiles(problem, z_width, x_variant, x_waves, y_coefs=None):
     an alternative built for the size, 6 or 8 (cf_problem_set_tiles); an
     unavailable choice raises and leaves the tiling as it was.  The x and z
     choices give identical results; the wall-normal layout agrees to
-    roundoff."""
+    roundoff.  The x choices take effect where the FP64 x pass is staged: in
+    pressure, and in the step of padded lengths without register radices."""
     v = X_VARIANTS.get(x_variant, x_variant)
     yk = get_tiles(problem)[4] if y_coefs is None else int(y_coefs)
     arr = (C.c_int * 5)(int(z_width), 0, int(v), int(x_waves), yk)
     _lib.check(_lib.load().cf_problem_set_tiles(problem.scheme.h, arr))
     return get_tiles(problem)
+
+
+def transforms(problem):
+    """Register radices of the step's x, z and y transforms, {"x": (r1, r2),
+    ...}; (0, 0): staged (cf_problem_transforms)."""
+    out = (C.c_int * 6)()
+    _lib.check(_lib.load().cf_problem_transforms(problem.scheme.h, out))
+    return {d: (out[2 * i], out[2 * i + 1]) for i, d in enumerate("xzy")}
 
 
 def last_gradient(scheme):

@@ -1680,10 +1680,11 @@ extern "C" int cf_random_state(cf_problem* h, double epsilon, unsigned long long
     return cf_pressure(h, U0, U1, U2, P, stream);
 }
 
-// Tile autotuner of one problem (FP64 step): times the z passes of the
-// nonlinear term for each in-place tile width and the x pass for each
-// wavefront count on the problem's workspaces, and keeps the fastest.  The
-// results of every pass do not depend on the tiling.
+// Tile autotuner of one problem, on its workspaces: times the z passes of the
+// nonlinear term for each tile width, the step's x pass where it is staged
+// (variants, wavefronts per block), the wall-normal layouts, and a mixed step's
+// FP32 x pass, and keeps the fastest.  The results of the x and z passes do not
+// depend on the tiling; the wall-normal layouts agree to roundoff.
 extern "C" int cf_problem_tune(cf_problem* h, void* stream) {
     if (!h) return fail(CF_ERR_ARGUMENT, "null problem");
     DeviceGuard dg(h->device);
@@ -1732,8 +1733,8 @@ extern "C" int cf_problem_tune(cf_problem* h, void* stream) {
     }
     h->KT = bestKT;
     h->zppt = bestPPT;
-    // x pass: wavefronts per block (even padded Nx), and for the rotating
-    // form the six-line or the split (three-line) variant
+    // staged x pass: wavefronts per block (even padded Nx), and for the
+    // rotating form the six-line, split (three-line) or async variant
     if (!rc && h->gd.Nxp % 2 == 0 && !h->xr1) {
         const int keepSplit = h->xsplit;
         int bestW[3] = {h->xwaves, h->xwavess, h->xwavesa}, bestSplit = keepSplit;
@@ -1839,7 +1840,7 @@ extern "C" int cf_problem_tiles(const cf_problem* h, int out[3]) {
     if (!h || !out) return fail(CF_ERR_ARGUMENT, "null argument");
     out[0] = h->KT;
     out[1] = h->zppt;
-    out[2] = h->xsplit == 2 ? h->xwavesa : h->xsplit ? h->xwavess : h->xwaves;  // of the x pass variant in use
+    out[2] = h->xsplit == 2 ? h->xwavesa : h->xsplit ? h->xwavess : h->xwaves;  // of the chosen staged x pass variant
     return CF_OK;
 }
 
@@ -1850,6 +1851,19 @@ extern "C" int cf_problem_get_tiles(const cf_problem* h, int tiles[5]) {
     tiles[2] = h->xsplit;
     tiles[3] = h->gd.Nxp % 2 ? 0 : h->xsplit == 2 ? h->xwavesa : h->xsplit ? h->xwavess : h->xwaves;
     tiles[4] = h->yk;
+    return CF_OK;
+}
+
+extern "C" int cf_problem_transforms(const cf_problem* h, int radices[6]) {
+    if (!h || !radices) return fail(CF_ERR_ARGUMENT, "null argument");
+    for (int i = 0; i < 6; ++i) radices[i] = 0;
+    if (h->mixed) return CF_OK;  // the FP32-mixed step runs the staged transforms
+    YArgs a;
+    std::memset(&a, 0, sizeof(a));
+    a.gd = h->gd;
+    y_reg_split(a, h->yl, h->yk);
+    const int r[6] = {h->xr1, h->xr2, h->zr1, h->zr2, a.r1, a.r2};
+    std::copy(r, r + 6, radices);
     return CF_OK;
 }
 

@@ -223,19 +223,25 @@ int cf_set_closure(cf_problem* h, cf_problem* helper, const float* theta, const 
 int cf_set_nonlinear(cf_problem* h, cf_forcing_fn fn, void* user, double* N0, double* N1, double* N2);
 
 /* Tile autotuner (no counterpart in the reference; a performance setting):
- * times the nonlinear term's z passes for each tile width and its x pass for
- * each variant and wavefront count on the problem's workspaces, on `stream`,
- * and keeps the fastest for the FP64 step (and, for a mixed-precision
- * problem, the fastest FP32 x pass of its step).  Results of every call are
- * identical for any tiling.  Synchronises the stream. */
+ * times the nonlinear term's z passes for each tile width, its x pass, where
+ * staged, for each variant and wavefront count, and the step's wall-normal
+ * kernels for each layout built, on the problem's workspaces, on `stream`,
+ * and keeps the fastest (for a mixed-precision problem also the fastest FP32
+ * x pass of its step).  Results are identical for any x and z tiling; the
+ * wall-normal layouts agree to roundoff, so a tuned step's last bits can
+ * depend on the layout that was fastest (set it with cf_problem_set_tiles for
+ * the same bits in every run).  Synchronises the stream. */
 int cf_problem_tune(cf_problem* h, void* stream);
-/* current tiles: out[0] z tile width, out[1] z in-place points per thread
- * (0: two buffers), out[2] x wavefronts per block */
+/* current tiles: out[0] z tile width, out[1] z in-place points per thread of
+ * the staged pass (0: two buffers), out[2] x wavefronts per block of the
+ * staged pass */
 int cf_problem_tiles(const cf_problem* h, int out[3]);
 
 /* Tile choice of the FP64 step, to read and to set (no counterpart in the
  * reference; lets a caller keep a tuning across runs, and the tests run every
- * variant): tiles[0] z tile width (1..min(32, Nx/2+1)), tiles[1] z in-place
+ * variant).  The x choices take effect where the FP64 x pass is staged: in
+ * cf_pressure, and in the step of padded lengths without register radices
+ * (cf_problem_transforms).  tiles[0] z tile width (1..min(32, Nx/2+1)), tiles[1] z in-place
  * points per thread (read only; set from the width), tiles[2] x pass variant
  * of the rotating form with even padded Nx (0 six LDS lines, 1 split: three
  * lines, velocity held in registers, 2 six lines with direct-to-LDS loads;
@@ -250,6 +256,12 @@ int cf_problem_tiles(const cf_problem* h, int out[3]);
  * unavailable choice returns CF_ERR_ARGUMENT and changes nothing. */
 int cf_problem_get_tiles(const cf_problem* h, int tiles[5]);
 int cf_problem_set_tiles(cf_problem* h, const int tiles[5]);
+
+/* Register radices of the step's transforms, two per direction: radices[0..1]
+ * x (padded Nx), [2..3] z (padded Nz; r2 = 1: the line in one lane), [4..5] y
+ * (2 Ny - 2, in the current wall-normal layout); 0 0: the staged transform
+ * (no such split, or a mixed-precision step). */
+int cf_problem_transforms(const cf_problem* h, int radices[6]);
 
 /* Uniform pressure gradient (dPdx, dPdz) returned by the last Stokes solve of
  * the last step (stokes.jl:101-107).  Synchronises the stream; HOST output. */
