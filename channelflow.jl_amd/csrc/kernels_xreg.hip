@@ -97,11 +97,10 @@ __device__ __forceinline__ double xrfma(double a, double b, double c) { return f
 struct XLines {
     const XArgs& a;
     double2* sm;
-    int N, nk, NL, slots;
+    int nk, NL, slots;
     unsigned ldk;
     long long gl0, nlines;
     __device__ __forceinline__ XLines(const XArgs& a_, double2* s, unsigned block) : a(a_), sm(s) {
-        N = a.gd.Nxp;
         nk = a.gd.nk;
         ldk = (unsigned)a.gd.ldk;
         NL = a.nl;
