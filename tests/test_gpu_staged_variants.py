@@ -87,3 +87,19 @@ def test_transforms_report(gpu):
     assert cf.transforms(prob) == {"x": (24, 8), "z": (16, 12), "y": (0, 0)}
     assert cf.transforms(_problem(cf, (22, 197, 8))) == {"x": (0, 0), "z": (12, 1), "y": (0, 0)}
     assert cf.transforms(_problem(cf, (32, 33, 32), precision="mixed")) == {"x": (0, 0), "z": (0, 0), "y": (0, 0)}
+
+
+def test_ensemble_of_unsplit_lengths(gpu):
+    import torch
+    cf = gpu
+    probs = [_problem(cf, (Nx, 9, 6)) for Nx in (216, 44, 32)]
+    states = [cf.perturbation_state(p, 0.05, seed=i) for i, p in enumerate(probs)]
+    own = [s.copy() for s in states]
+    for p, s in zip(probs, own):
+        cf.step_(p.scheme, p.nlterm, s.velocity, s.stagepressure, 0.0, nsteps=3, **p.constraint)
+    for tune in (False, True):
+        runs = [s.copy() for s in states]
+        cf.Ensemble(probs, runs, tune=tune).advance(3)
+        torch.cuda.synchronize()
+        for a, b in zip(runs, own):
+            assert torch.equal(a.velocity, b.velocity) and torch.equal(a.stagepressure, b.stagepressure), tune
