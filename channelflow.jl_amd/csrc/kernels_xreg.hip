@@ -20,9 +20,9 @@
 // The staged form (a wavefront per line, half-length lines in LDS) issued 243
 // 16-byte LDS operations a line, about 60 of its 91 us at 128x97x128 at the
 // full LDS rate.  Rotating form, us a launch, staged -> here: 32x33x32 11.3 ->
-// 4.7, 64x65x64 33.6 -> 13.4, 128x97x128 91 -> 52.2 (3.3 TB/s), 256x257x256
+// 4.7, 64x65x64 33.6 -> 13.0, 128x97x128 91 -> 52.2 (3.3 TB/s), 256x257x256
 // 1030 -> 566 (3.2 TB/s); 42x49x54, whose odd padded length runs the block-wide
-// staged pass, 130 -> 7.0; convective 80x65x96 74.5 -> 39.1.  Bound by HBM at
+// staged pass, 130 -> 7.0; convective 80x65x96 74.5 -> 33.0.  Bound by HBM at
 // 128x97x128 and above (a device copy takes 35 us for those bytes).
 #include <algorithm>
 
@@ -56,9 +56,13 @@ __host__ __device__ constexpr int xr_pitch(int r2) { return (r2 / 2 + 1) | 1; }
 
 // Split N = a b, a = R1 and b = R2: b bounds the registers of phase B (six real
 // lines of b points: 192 registers at 16, the largest built), a those of phases
-// A and C.  Of the splits with radices built, the one nearest to a = 2.5 b: the
-// lanes of the three phases (3 b + 6, a and 1.5 b + 3 of the rotating form)
-// are alike there.
+// A and C.  Of the splits with radices built, the one nearest to a = 2 b, where
+// the lanes of the phases (3 b + 6, a and 1.5 b + 3 of the rotating form) are
+// closest; of two as near, the one with a <= 12, whose kernel needs about half
+// the registers, else the larger a.  Steps of Nx x 33 x 96, us, rotating and
+// convective: N = 96 as 16 x 6 218 and 242, as 12 x 8 213 and 225; 108 as 18 x 6
+// 223 and 256, as 12 x 9 218 and 232; 192 as 24 x 8 261 and 295, as 16 x 12 260
+// and 302; 216 as 24 x 9 271 and 308, as 18 x 12 275 and 323.
 __host__ __device__ constexpr bool xr_r1(int r) {
     return (r >= 2 && r <= 10) || r == 12 || (r >= 14 && r <= 16) || r == 18 || r == 20 || r == 21 || r == 24;
 }
@@ -72,11 +76,11 @@ __host__ __device__ constexpr int xr_split(int n) {  // R2, 0: none
             best = b;
             continue;
         }
-        // max(a / 2.5 b, 2.5 b / a) of both, cross-multiplied
+        // max(a / 2 b, 2 b / a) of both, cross-multiplied
         const int a0 = n / best;
-        const long long nu = 2 * a > 5 * b ? 2 * a : 5 * b, de = 2 * a > 5 * b ? 5 * b : 2 * a;
-        const long long nu0 = 2 * a0 > 5 * best ? 2 * a0 : 5 * best, de0 = 2 * a0 > 5 * best ? 5 * best : 2 * a0;
-        if (nu * de0 < nu0 * de) best = b;
+        const long long nu = a > 2 * b ? a : 2 * b, de = a > 2 * b ? 2 * b : a;
+        const long long nu0 = a0 > 2 * best ? a0 : 2 * best, de0 = a0 > 2 * best ? 2 * best : a0;
+        if (nu * de0 < nu0 * de || (nu * de0 == nu0 * de && a <= 12 && a0 > 12)) best = b;
     }
     return best;
 }
